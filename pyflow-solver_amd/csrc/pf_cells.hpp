@@ -51,6 +51,29 @@ __device__ inline T lap_coherent5(T c, T e, T w, T n, T s, int nx, int ny, int j
   return (T(0) + xp) + yp;
 }
 
+// Division of many numerators by one spacing b > 0, correctly rounded like the
+// hardware's IEEE division but in three operations instead of its dozen
+// (scale, reciprocal estimate, refinement, fix-up). With y = RN(1/b):
+//   q = RN(a y),  t = RN(q b - a),  q' = RN(q - t y)   (fused multiply-adds)
+// (Markstein 1990; for divisors known in advance Brisebarre, Muller & Raina,
+// IEEE Trans. Comput. 53(8), 2004). q' can differ from RN(a/b) only where a/b
+// lies within a few units of 2^-106 of a midpoint between two doubles; for a
+// given b these numerators can be enumerated, and divisor_exact() (host) tries
+// each of them, so `fast` is set only for divisors on which q' is RN(a/b) for
+// every a in the range below. t keeps the sign of a zero numerator (-0/b = -0).
+struct DivBy {
+  double b, y;  // the spacing and RN(1/b)
+};
+__device__ __host__ inline double div_fast(double a, const DivBy& d) {
+  const double q = a * d.y;
+  const double t = fma(q, d.b, -a);
+  return fma(-t, d.y, q);
+}
+// With b in [2^-64, 2^64], zeros and every |a| >= 2^-800 divide exactly that way,
+// up to magnitudes where q overflows, and there (and for Inf and NaN) q' is not
+// finite. A caller sends smaller numerators and results that are not finite
+// through the division itself.
+
 // Pressure operators (pressure_solver.py:97-105 and :69-77).
 //   op 0: -lap, row 0 replaced by the identity (pinned reference cell)
 //   op 1: +lap, every boundary row replaced by the identity (Dirichlet)

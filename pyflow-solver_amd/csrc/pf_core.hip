@@ -78,7 +78,7 @@ struct pf_batch {
   PfCav* dcav = nullptr;
   PfScal* dscal = nullptr;
   int* dtile = nullptr;  // workgroup -> cavity slot
-  int* dactive = nullptr;
+  int* dactive = nullptr;  // cavities still running; whether a resident solve gave up waiting
   PfScal* hscal = nullptr;  // pinned mirror
   int* hactive = nullptr;   // pinned
   int total_blocks = 0;
@@ -89,6 +89,13 @@ struct pf_batch {
   int xd_kinds = 0;      // rounds of those cavities: bit 0 one PCG iteration, bit 1 two
   bool multi = false;    // some cavity has several regions per workgroup
   bool occ2 = false;     // every cavity fits the two-workgroups-per-CU kernel
+  int res_kind = 0;      // rounds with resident solves: 0 none, 1 FP64 (k_round_res64)
+  char* dres = nullptr;  // their exchange buffers (KArgs::res), allocated when first used
+  size_t dres_bytes = 0;
+  bool res_ready = false;  // dres holds its resting values
+  bool res_on = false;     // rounds queued now may run resident solves
+  int num_cu = 0;
+  int meet_ticks = 20000;  // KArgs::meet_ticks: 200 us unless PYFLOW_MEET_US says otherwise
   bool s3 = false;       // every cavity runs three PCG iterations per round (k_round_ca3)
   bool tables_dirty = true;
   int graph_len = 0;                      // rounds per captured graph (even; 0: direct launches)
@@ -219,6 +226,47 @@ static int lds_floats_of(const PfCav& c) {
   return c.ca == 2 ? ca3_lds_floats(c.tpb) : (c.ca ? ca_lds_floats(c.tpb) : region_lds_floats(c.tpb));
 }
 
+// Whether div_fast(a, {b, RN(1/b)}) is RN(a/b) for every a in its range (see
+// DivBy). Scaled to a, b in [1, 2) with 53-bit integers A, B, a quotient in
+// [2^e, 2^(e+1)), e = 0 or -1, has its midpoints at M 2^-53 2^e with M odd in
+// [2^53, 2^54), and a/b lies off one by D / (b 2^(105 - e)) with the integer
+// D = A 2^(53 - e) - B M. The method's error before its last rounding is at
+// most 2^-105 (e = 0; q is off by at most 2^-52, RN(1/b) by 2^-54) or
+// 3.5 2^-106 (e = -1, where t may round as well), so only |D| <= 7 could
+// round the wrong way. For each such D the congruence B M = -D mod 2^(53 - e)
+// gives every M, hence every candidate A, and each is divided both ways.
+// Divisors outside [2^-64, 2^64] are refused.
+static bool divisor_exact(double b) {
+  if (!(b >= 0x1p-64 && b <= 0x1p64)) return false;
+  int ex;
+  const double fb = 2.0 * std::frexp(b, &ex);  // in [1, 2)
+  const uint64_t B = (uint64_t)(fb * 0x1p52);
+  const DivBy d{fb, 1.0 / fb};
+  int t = 0;
+  while (!((B >> t) & 1)) ++t;
+  const uint64_t odd = B >> t;
+  uint64_t inv = odd;  // inverse of `odd` mod 2^64 (Newton)
+  for (int k = 0; k < 6; ++k) inv *= 2 - odd * inv;
+  for (int e = 0; e >= -1; --e) {
+    const int sh = 53 - e;  // A 2^sh = B M + D
+    for (int64_t D = -8; D <= 8; ++D) {
+      if (D == 0 || (D & (((int64_t)1 << t) - 1))) continue;  // 2^t divides A 2^sh - B M
+      const uint64_t step = (uint64_t)1 << (sh - t);
+      const uint64_t m0 = ((uint64_t)(-(D / ((int64_t)1 << t))) * inv) & (step - 1);
+      for (uint64_t M = m0; M < ((uint64_t)1 << 54); M += step) {
+        if (M < ((uint64_t)1 << 53) || !(M & 1)) continue;
+        const __int128 num = (__int128)B * M + D;
+        const uint64_t A = (uint64_t)(num >> sh);
+        if (A < ((uint64_t)1 << 52) || A >= ((uint64_t)1 << 53)) continue;
+        const double a = (double)A * 0x1p-52;
+        if ((e == 0) != (a >= fb)) continue;
+        if (div_fast(a, d) != a / fb) return false;
+      }
+    }
+  }
+  return true;
+}
+
 static void fill_params(PfCav& c, const pf_cavity_params* p, int prec) {
   c.nx = p->nx;
   c.ny = p->ny;
@@ -235,6 +283,12 @@ static void fill_params(PfCav& c, const pf_cavity_params* p, int prec) {
   c.mode = p->mode;
   c.prec = prec;
   c.lid = p->lid_velocity;
+  // PYFLOW_FASTDIV=0 keeps true divisions. divisor_exact runs once per new
+  // spacing (the drop-in loop sets its parameters before every step).
+  if (prec == PF_PREC_FP64 && (c.rdx == 0.0 || c.dx != p->dx || c.dy != p->dy))
+    c.fastdiv = (env_switch("PYFLOW_FASTDIV", 1) != 0 && divisor_exact(p->dx) && divisor_exact(p->dy)) ? 1 : 0;
+  c.rdx = 1.0 / p->dx;
+  c.rdy = 1.0 / p->dy;
   c.dx = p->dx;
   c.dy = p->dy;
   c.nu = p->nu;
@@ -275,6 +329,34 @@ static void fill_params(PfCav& c, const pf_cavity_params* p, int prec) {
 static bool same_operator(const PfCav& a, const PfCav& b) { return a.op == b.op && a.dx == b.dx && a.dy == b.dy; }
 
 static void drop_graphs(pf_batch* b);
+
+// Batches whose rounds may run a solve by resident workgroups: one FP64
+// cavity with one region of at most 4 tiles per workgroup and no more
+// workgroups than CUs, so that all of them can be on the GPU at once
+// (PYFLOW_RESIDENT=0: never). Results are bitwise the same either way.
+static int resident_kind(const pf_batch* b) {
+  if (b->single_slot < 0 || env_switch("PYFLOW_RESIDENT", 1) == 0) return 0;
+  const PfCav& c = b->hcav[b->single_slot];
+  if (c.rpw != 1 || c.tpb > 4 || c.nblk > std::min(b->num_cu, kResMaxBlk)) return 0;
+  if (c.nblk == 1 && !c.local) return 0;  // PYFLOW_LOCAL=0: one phase per launch
+  return b->prec == PF_PREC_FP64 ? 1 : 0;
+}
+
+// Runs (pf_batch_run, pf_batch_launch) let a launch run a whole solve; served
+// batches (pf_batch_advance) keep one phase per launch, so that a chunk of
+// rounds is short whatever the solves need. Puts the exchange buffers into
+// their resting state before the first use.
+static int set_resident(pf_batch* b, bool on) {
+  on = on && b->res_kind != 0;
+  if (on != b->res_on) drop_graphs(b);  // their nodes carry KArgs::res
+  if (on && (!b->res_on || !b->res_ready)) {
+    HIPCHK(hipMemsetAsync(b->dres, 0xff, b->dres_bytes, b->stream));
+    HIPCHK(hipMemsetAsync(b->dres + kResMeet, 0, 256, b->stream));
+    b->res_ready = true;
+  }
+  b->res_on = on;
+  return PF_OK;
+}
 
 static int sync_tables(pf_batch* b) {
   if (!b->tables_dirty) return PF_OK;
@@ -319,6 +401,18 @@ static int sync_tables(pf_batch* b) {
       b->occ2 = b->occ2 && c.ca == 1 && !c.xd && c.tpb <= 2 && c.rpw == 1;
       b->multi = b->multi || b->hcav[s].rpw > 1;
     }
+  b->res_kind = resident_kind(b);
+  b->res_ready = false;
+  if (b->res_kind) {
+    const size_t need = res64_bytes(b->hcav[b->single_slot].nblk);
+    if (b->dres_bytes < need) {
+      if (b->dres) HIPCHK(hipFree(b->dres));
+      b->dres = nullptr;
+      b->dres_bytes = 0;
+      HIPCHK(hipMalloc((void**)&b->dres, need));
+      b->dres_bytes = need;
+    }
+  }
   HIPCHK(hipMemcpyAsync(b->dcav, b->hcav.data(), sizeof(PfCav) * b->max_cav, hipMemcpyHostToDevice, b->stream));
   if (!tiles.empty())
     HIPCHK(hipMemcpyAsync(b->dtile, tiles.data(), sizeof(int) * tiles.size(), hipMemcpyHostToDevice, b->stream));
@@ -404,6 +498,10 @@ static RoundLaunch round_launch(const pf_batch* b) {
     L.fn = b->unroll >= 4 ? round_fn_u<double, 4>(b) : b->unroll == 2 ? round_fn_u<double, 2>(b)
                                                                       : round_fn_u<double, 1>(b);
     L.lds = (size_t)b->lds_floats * sizeof(float);
+    if (b->res_kind == 1) {
+      L.fn = (const void*)k_round_res64;
+      L.lds = std::max(L.lds, res64_lds_doubles(b->hcav[b->single_slot].tpb) * sizeof(double));
+    }
   }
   return L;
 }
@@ -418,6 +516,8 @@ static KArgs round_args(const pf_batch* b, int parity) {
   K.max_cav = b->max_cav;
   K.parity = parity;
   K.slot0 = b->single_slot;
+  K.res = b->res_on ? b->dres : nullptr;
+  K.meet_ticks = b->meet_ticks;
   if (b->single_slot >= 0) K.cav0 = b->hcav[b->single_slot];
   return K;
 }
@@ -750,18 +850,20 @@ int pf_batch_create_empty(int precision, int max_cav, int64_t max_tiles, void* s
   // (empty rounds). 1024 against 256 made the 200 steps of the 1024^2 cavity
   // 0.6% faster before that run was tracked. A tracked run (one cavity, several
   // steps) queues at most max_ahead rounds on a prediction (tracked_chunk).
+  b->meet_ticks = 100 * std::max(0, std::min(1000000, env_switch("PYFLOW_MEET_US", 200)));
   b->max_chunk = std::max<int64_t>(16, env_int("PYFLOW_MAX_CHUNK", 1024));
   b->track = env_switch("PYFLOW_TRACK", 1) != 0;
   b->max_ahead = std::max<int64_t>(16, env_int("PYFLOW_MAX_AHEAD", 4096));
   b->used.assign(max_cav, 0);
   b->dreset.assign(max_cav, 0);
   hipError_t e = hipGetDevice(&b->device);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&b->num_cu, hipDeviceAttributeMultiprocessorCount, b->device);
   if (e == hipSuccess) e = hipMalloc((void**)&b->dcav, sizeof(PfCav) * max_cav);
   if (e == hipSuccess) e = hipMalloc((void**)&b->dscal, 2 * sizeof(PfScal) * max_cav);
   if (e == hipSuccess) e = hipMalloc((void**)&b->dtile, sizeof(int) * max_tiles);
-  if (e == hipSuccess) e = hipMalloc((void**)&b->dactive, sizeof(int));
+  if (e == hipSuccess) e = hipMalloc((void**)&b->dactive, 2 * sizeof(int));
   if (e == hipSuccess) e = hipHostMalloc((void**)&b->hscal, sizeof(PfScal) * max_cav, hipHostMallocDefault);
-  if (e == hipSuccess) e = hipHostMalloc((void**)&b->hactive, sizeof(int), hipHostMallocDefault);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&b->hactive, 2 * sizeof(int), hipHostMallocDefault);
   if (e == hipSuccess) e = hipHostMalloc((void**)&b->hobs, sizeof(PfScal), hipHostMallocDefault);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ev, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreate(&b->ev_t0);
@@ -772,10 +874,10 @@ int pf_batch_create_empty(int precision, int max_cav, int64_t max_tiles, void* s
     return fail(PF_ENOMEM, msg);
   }
   std::memset(b->hscal, 0, sizeof(PfScal) * max_cav);
-  *b->hactive = 0;
+  b->hactive[0] = b->hactive[1] = 0;
   e = hipMemsetAsync(b->dscal, 0, 2 * sizeof(PfScal) * max_cav, b->stream);
   if (e == hipSuccess) e = hipMemsetAsync(b->dtile, 0xff, sizeof(int) * max_tiles, b->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(b->dactive, 0, sizeof(int), b->stream);
+  if (e == hipSuccess) e = hipMemsetAsync(b->dactive, 0, 2 * sizeof(int), b->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
   if (e != hipSuccess) {
     std::string msg = std::string("init failed: ") + hipGetErrorString(e);
@@ -897,6 +999,7 @@ int pf_batch_destroy(pf_batch* b) {
   if (b->dscal) (void)hipFree(b->dscal);
   if (b->dtile) (void)hipFree(b->dtile);
   if (b->dactive) (void)hipFree(b->dactive);
+  if (b->dres) (void)hipFree(b->dres);
   if (b->hscal) (void)hipHostFree(b->hscal);
   if (b->hactive) (void)hipHostFree(b->hactive);
   if (b->hobs) (void)hipHostFree(b->hobs);
@@ -1112,10 +1215,13 @@ static int arm(pf_batch* b, int nsteps, const int32_t* active) {
     guard = std::max(guard, (int64_t)sc.steps_left * per + setup + 64);
     ++nact;
   }
-  *b->hactive = nact;
+  b->hactive[0] = nact;
+  b->hactive[1] = 0;
+  rc = set_resident(b, true);
+  if (rc) return rc;
   int rc2 = push_scal_all(b);
   if (rc2) return rc2;
-  HIPCHK(hipMemcpyAsync(b->dactive, b->hactive, sizeof(int), hipMemcpyHostToDevice, b->stream));
+  HIPCHK(hipMemcpyAsync(b->dactive, b->hactive, 2 * sizeof(int), hipMemcpyHostToDevice, b->stream));
   HIPCHK(hipStreamSynchronize(b->stream));
   b->rounds = 0;
   b->round_guard = guard;
@@ -1132,7 +1238,7 @@ static int chunk(pf_batch* b, int64_t n) {
     HIPCHK(hipEventRecord(b->ev_t1, b->stream));
     b->timed_rounds += n;
   }
-  HIPCHK(hipMemcpyAsync(b->hactive, b->dactive, sizeof(int), hipMemcpyDeviceToHost, b->stream));
+  HIPCHK(hipMemcpyAsync(b->hactive, b->dactive, 2 * sizeof(int), hipMemcpyDeviceToHost, b->stream));
   if (b->obs_slot >= 0) {
     const int par = (int)((b->round + 1) & 1);  // buffer of the last round
     HIPCHK(hipMemcpyAsync(b->hobs, b->dscal + (size_t)par * b->max_cav + b->obs_slot, sizeof(PfScal),
@@ -1141,6 +1247,12 @@ static int chunk(pf_batch* b, int64_t n) {
   HIPCHK(hipEventRecord(b->ev, b->stream));
   b->chunk_pending = true;
   return PF_OK;
+}
+
+// A resident solve waited kWaitTicks for a workgroup that was running.
+static int resident_failed(pf_batch* b) {
+  b->res_ready = false;
+  return fail(PF_ESTATE, "a resident solve stopped waiting for its workgroups (internal error)");
 }
 
 // Rounds to queue next in a tracked run (one cavity stepping nsteps > 1 steps),
@@ -1189,6 +1301,7 @@ int pf_batch_run(pf_batch* b, int nsteps, const int32_t* active, pf_step_diag* d
         HIPCHK(hipEventElapsedTime(&ms, b->ev_t0, b->ev_t1));
         b->gpu_ms += ms;
       }
+      if (b->hactive[1]) return resident_failed(b);
       if (*b->hactive <= 0) break;
       if (b->rounds > b->round_guard) return fail(PF_ESTATE, "round limit exceeded (internal error)");
       const int64_t n = (b->obs_slot >= 0) ? tracked_chunk(b, over, nsteps) : step;
@@ -1247,6 +1360,7 @@ int pf_batch_poll(pf_batch* b, int* done) {
     *done = 1;
     return PF_OK;
   }
+  if (b->hactive[1]) return resident_failed(b);
   if (*b->hactive <= 0) {
     int rc = pull_scal(b);
     if (rc) return rc;
@@ -1300,7 +1414,7 @@ int pf_batch_start(pf_batch* b, int slot, int nsteps) {
   rc = push_scal(b, slot);
   if (rc) return rc;
   *b->hactive += 1;
-  HIPCHK(hipMemcpyAsync(b->dactive, b->hactive, sizeof(int), hipMemcpyHostToDevice, b->stream));
+  HIPCHK(hipMemcpyAsync(b->dactive, b->hactive, 2 * sizeof(int), hipMemcpyHostToDevice, b->stream));
   HIPCHK(hipStreamSynchronize(b->stream));
   b->serving = true;
   return PF_OK;
@@ -1313,6 +1427,8 @@ int pf_batch_advance(pf_batch* b, int64_t rounds) {
   if (rc) return rc;
   b->serving = true;
   b->obs_slot = -1;
+  rc = set_resident(b, false);
+  if (rc) return rc;
   if (b->total_blocks <= 0) return PF_OK;
   return chunk(b, rounds);
 }

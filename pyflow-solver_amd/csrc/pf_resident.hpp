@@ -1,0 +1,536 @@
+// Resident solves: the CG iterations of one cavity run inside one launch, its
+// workgroups exchanging partial sums and region edges through memory.
+//
+// Protocol
+// --------
+// A cavity of at most one region per workgroup and at most one workgroup per
+// CU can have all its workgroups on the GPU at once. When a solve's CG phase
+// begins, its workgroups first meet (resident_enter): each adds itself to the
+// launch's arrival word. If all arrive within KArgs::meet_ticks every workgroup is
+// known to be running and the solve goes on in this launch; if one of them
+// times out first (the GPU is shared with other work) it marks the word, all
+// of them see the mark, and the launch runs one ordinary round, like a launch
+// without this path. Afterwards each wait is for a workgroup that is running,
+// so it ends; all are bounded by kWaitTicks nevertheless, after which the
+// launch gives up and reports an error.
+//
+// Nothing is fenced. Values cross between workgroups only through relaxed
+// device-scope atomic loads and stores, which reach past the per-XCD L2s, and
+// every value that is waited for announces itself:
+//   partial sums  64-bit words that hold kSent (all ones) until their writer
+//                 stores the sum; workgroup 0 collects them, folds them as the
+//                 next round would, runs the tail, and puts kSent back. Two
+//                 buffers alternate, so a word is reset long before it is
+//                 written again;
+//   tail results  words of 32 bits of payload and a 32-bit sequence number,
+//                 stored by workgroup 0 on kCopies lines (fewer readers per line);
+//   region edges  one inbox per region side, read by that region only, which
+//                 puts kSent back; two buffers alternate here too.
+// A sum or cell that equals kSent (a NaN) is stored as another NaN.
+#pragma once
+
+namespace pf {
+
+constexpr unsigned long long kSent = ~0ull;
+constexpr unsigned long long kOtherNan = 0x7ff8000000000000ull;
+constexpr int kCopies = 8;
+constexpr int kResMaxBlk = 256;           // workgroups of a resident cavity
+constexpr long long kWaitTicks = 1000000000;  // 10 s
+constexpr int kResIters = 4096;           // CG iterations per launch at most
+constexpr double kTinyD = 0x1p-300;
+constexpr unsigned kMeetAbort = 0x10000u;
+
+// Layout of KArgs::res (bytes; every block starts on a 128-byte line).
+constexpr size_t kResMeet = 0;             // arrival words, one per round parity, 128 bytes apart
+constexpr size_t kResBcast = 512;          // kCopies lines of 16 words
+constexpr size_t kResPart = 4096;          // 2 x 3 x kResMaxBlk words
+constexpr size_t kResInbox = kResPart + 2 * 3 * kResMaxBlk * 8;  // [2][nblk][4 sides][64] words
+__host__ __device__ constexpr size_t res64_bytes(int nblk) { return kResInbox + (size_t)2 * nblk * 4 * 64 * 8; }
+enum { SIDE_W = 0, SIDE_E = 1, SIDE_S = 2, SIDE_N = 3 };
+
+constexpr int kResPitch = TX + 3;  // LDS pitch of the FP64 direction: 64 columns, a ring, odd
+__host__ __device__ constexpr int res64_lds_doubles(int m) { return (TY * m + 2) * kResPitch; }
+
+__device__ inline void dev_store(unsigned long long* p, unsigned long long v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline unsigned long long dev_load(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void dev_store_f64(unsigned long long* p, double v) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  dev_store(p, u == kSent ? kOtherNan : u);
+}
+// Every memory operation of this wave has completed.
+__device__ inline void drain_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Words the workgroup shares during a resident solve; they overlay the
+// reduction array, which the solve does not use.
+struct ResShared {
+  double val[4];        // alpha, or beta
+  double wsum[3][NWAVE];  // wave totals: P, and the two of Q
+  unsigned seq0;        // sequence number of the last broadcast before this launch
+  int go, dead;
+  int tiny[2];  // some d of the region or its ring is a tiny number, by iteration parity
+};
+static_assert(sizeof(ResShared) <= sizeof(double) * NWAVE * NPS, "ResShared overlays the reduction array");
+
+// Whether this launch's workgroups are all running (see above). Every thread
+// of every workgroup of the cavity calls it once per launch at most.
+__device__ inline bool resident_enter(const KArgs& KA, const PfCav& C, int b, ResShared* sh) {
+  if (KA.res == nullptr) return false;
+  const int nblk = C.nblk;
+  __syncthreads();  // the preamble's use of the overlaid array has ended
+  if (tid_flat() == 0) {
+    sh->dead = 0;
+    sh->go = 1;
+    sh->tiny[0] = sh->tiny[1] = 0;
+    if (nblk > 1) {
+      unsigned* meet = (unsigned*)(KA.res + kResMeet + 128 * KA.parity);
+      const unsigned long long* line =
+          (const unsigned long long*)(KA.res + kResBcast) + 16 * (b & (kCopies - 1));
+      sh->seq0 = (unsigned)(dev_load(line) >> 32);
+      drain_vmem();  // read before arriving: workgroup 0 broadcasts only after every arrival
+      const long long t0 = wall_clock64();
+      unsigned cur = __hip_atomic_fetch_add(meet, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+      while (true) {
+        if (cur & kMeetAbort) {
+          sh->go = 0;
+          break;
+        }
+        if (cur == (unsigned)nblk) break;
+        if (wall_clock64() - t0 > KA.meet_ticks) {
+          unsigned want = cur | kMeetAbort;
+          if (__hip_atomic_compare_exchange_strong(meet, &cur, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT)) {
+            sh->go = 0;
+            break;
+          }
+          continue;  // cur holds the word that won
+        }
+        __builtin_amdgcn_s_sleep(1);
+        cur = __hip_atomic_load(meet, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+  }
+  __syncthreads();
+  return sh->go != 0;
+}
+// The previous launch's arrival word, for the launch after this one.
+__device__ inline void resident_clear_meet(const KArgs& KA) {
+  if (KA.res != nullptr)
+    __hip_atomic_store((unsigned*)(KA.res + kResMeet + 128 * (KA.parity ^ 1)), 0u, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Word `lane` (0 .. nw-1) of the broadcast with sequence number `seq`, polled
+// by one whole wave. False after kWaitTicks.
+__device__ inline bool bcast_wait(const unsigned long long* line, int lane, int nw, unsigned seq, unsigned& payload) {
+  const long long t0 = wall_clock64();
+  while (true) {
+    const unsigned long long w = (lane < nw) ? dev_load(line + lane) : ((unsigned long long)seq << 32);
+    payload = (unsigned)w;
+    if (!__any((unsigned)(w >> 32) != seq)) return true;
+    if (wall_clock64() - t0 > kWaitTicks) return false;
+  }
+}
+// The value of kSent-marked words q = lane + 64 t (t < 4, q < n), polled by one
+// whole wave; consumed words get kSent back. False after kWaitTicks.
+__device__ inline bool words_take(unsigned long long* w, int lane, int n, double (&v)[4]) {
+  const long long t0 = wall_clock64();
+  unsigned long long x[4];
+  while (true) {
+    bool miss = false;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int q = lane + 64 * t;
+      x[t] = (q < n) ? dev_load(w + q) : 0ull;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) miss |= x[t] == kSent;
+    if (!__any(miss)) break;
+    if (wall_clock64() - t0 > kWaitTicks) return false;
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int q = lane + 64 * t;
+    if (q < n) dev_store(w + q, kSent);
+    v[t] = __longlong_as_double((long long)x[t]);
+  }
+  return true;
+}
+// The fold of a round's preamble: per lane in increasing workgroup order, then
+// the DPP tree; the total is broadcast from lane 63.
+__device__ inline double fold_words(int lane, int n, const double (&v)[4]) {
+  double a = 0.0;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    if (lane + 64 * t < n) a = a + v[t];
+  a = wave_reduce<false>(a);
+  const long long bits = __double_as_longlong(a);
+  const int lo = __builtin_amdgcn_readlane((int)(bits & 0xffffffffll), 63);
+  const int hi = __builtin_amdgcn_readlane((int)(bits >> 32), 63);
+  return __longlong_as_double((long long)(unsigned)lo | ((long long)hi << 32));
+}
+// The sum of the wave totals in wave order (block_partials_k's fold).
+__device__ inline double fold_waves(const double* w) {
+  double t = w[0];
+#pragma unroll
+  for (int k = 1; k < NWAVE; ++k) t = t + w[k];
+  return t;
+}
+
+// The CG iterations of an FP64 solve (phases P and Q of chunk_p / chunk_q and
+// their tails), from a P phase to the end of the solve or kResIters of them.
+// A thread keeps x, r, d and q = A d of its M cells in registers; d is also in
+// LDS with a one-cell ring, where the stencil reads it. A region's ring of r is
+// received from its neighbours after every Q, and the ring's d is formed from
+// it by the owner's expression, so it carries the owner's bits. Cell
+// expressions, per-thread sums, block reduction, fold and tails are those of
+// the rounds, in their order: the results are the bits of one launch per
+// phase. What bounds it is the chain of an iteration: two sums over all
+// workgroups (about 2 us each from the first store to the last reader; one
+// launch per phase spends 2.5 us between kernels and as much again on the
+// state, the partials and the vectors), the stencil with its six divisions, and
+// four barriers. Per iteration, one launch per phase -> resident: 5.4 -> 3.8 us
+// at 64^2 (one workgroup, against local_cg), 26 -> 9.0 us at 130x97,
+// 23.2 -> 9.6 us at 512^2, 27.3 -> 10.1 us at 1000x700 (176 workgroups). The
+// state is left as after a Q round's tail. A NaN residual leaves
+// the loop (such a solve goes on one phase per launch, where a host that looks
+// for NaN sees it). One workgroup: no exchange at all, every thread forms the
+// tails' scalars from the wave totals.
+template <int M>
+__device__ __attribute__((always_inline)) inline void resident_cg64(const KArgs& KA, const PfCav& C, PfScal& st,
+                                                                    double (*sm)[NPS], double* __restrict__ lD, int b) {
+  ResShared& sh = *(ResShared*)sm;
+  constexpr int P = kResPitch;
+  const int nx = C.nx, ny = C.ny, nblk = C.nblk, tiles_x = C.tiles_x;
+  const int li = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);  // = the row within a tile
+  const int rx = b % tiles_x, ry = b / tiles_x;
+  const int i0 = rx * TX, j0 = ry * TY * M;
+  const int i = i0 + li;
+  const bool multi = nblk > 1;
+  const bool full = (i0 + TX <= nx) && (j0 + TY * M <= ny);
+  const int op = C.op;
+  const DivBy dx{C.dx, C.rdx}, dy{C.dy, C.rdy};
+  const bool fast = C.fastdiv != 0;
+  const double sign = (op == 0) ? -1.0 : 1.0;
+  const int maxiter = C.maxiter;
+  const double atol = st.inner_atol;
+  double* X = (double*)C.x;
+  double* R = (double*)C.r;
+  double* const D0 = (double*)C.d0;
+  double* const D1 = (double*)C.d1;
+  int it = st.it, it_total = st.it_total;
+  double rho = st.rho, beta = st.beta;
+
+  // LDS word of cell (16 m + wave, li) and of its neighbours; a missing
+  // neighbour is the cell itself, whose difference is +0 as the operator has it.
+  const int c0 = (wave + 1) * P + li + 1;
+  const int oE = c0 + ((i + 1 < nx) ? 1 : 0), oW = c0 - ((i > 0) ? 1 : 0);
+  int oN[M], oS[M];
+  double xv[M], rv[M], dv[M], qv[M], wv[M];
+  bool in[M];
+  unsigned idm = 0;  // identity rows among the thread's cells
+  {
+    const double* Dold = (it & 1) ? D0 : D1;
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const int j = j0 + TY * m + wave;
+      in[m] = (i < nx) && (j < ny);
+      const size_t k = in[m] ? (size_t)j * nx + i : 0;
+      const double xx = X[k], rr = R[k], dd = Dold[k];
+      xv[m] = in[m] ? xx : 0.0;
+      rv[m] = in[m] ? rr : 0.0;
+      dv[m] = in[m] ? dd : 0.0;
+      wv[m] = jacobi_minv(C.jacobi, C.invd, nx, ny, j, i);
+      const int o = c0 + TY * m * P;
+      oN[m] = o + ((j + 1 < ny) ? P : 0);
+      oS[m] = o - ((j > 0) ? P : 0);
+      const bool id = (op == 0) ? (j == 0 && i == 0) : (j == 0 || j == ny - 1 || i == 0 || i == nx - 1);
+      if (id && in[m]) idm |= 1u << m;
+    }
+  }
+  const bool any_id = __any(idm != 0);
+  // Ring: wave 4 + side holds that side's cells, one per lane.
+  const int side = wave - 4;
+  bool ring = false;
+  double rr = 0.0, rd = 0.0, rw = 0.0;
+  int ro = 0;
+  unsigned long long* inbox = (unsigned long long*)(KA.res + kResInbox);
+  unsigned long long* mine = inbox;
+  if (multi && side >= 0 && side < 4) {
+    int gi, gj, row, col;
+    if (side < 2) {
+      gi = side == SIDE_W ? i0 - 1 : i0 + TX;
+      gj = j0 + li;
+      row = li + 1;
+      col = side == SIDE_W ? 0 : TX + 1;
+      ring = li < TY * M;
+    } else {
+      gi = i0 + li;
+      gj = side == SIDE_S ? j0 - 1 : j0 + TY * M;
+      row = side == SIDE_S ? 0 : TY * M + 1;
+      col = li + 1;
+      ring = true;
+    }
+    ring = ring && gi >= 0 && gi < nx && gj >= 0 && gj < ny;
+    ro = ring ? row * P + col : 0;
+    const size_t k = ring ? (size_t)gj * nx + gi : 0;
+    const double* Dold = (it & 1) ? D0 : D1;
+    rr = R[k];
+    rd = Dold[k];
+    rw = jacobi_minv(C.jacobi, C.invd, nx, ny, gj, gi);
+    mine = inbox + ((size_t)b * 4 + side) * 64 + li;
+  }
+  const size_t inbuf = (size_t)nblk * 4 * 64;  // words per inbox buffer
+  // Inboxes this thread's edge cells go to: columns (lanes 0 and 63), rows.
+  const bool sendW = multi && li == 0 && rx > 0, sendE = multi && li == TX - 1 && i0 + TX < nx;
+  const bool sendS = multi && wave == 0 && j0 > 0, sendN = multi && wave == TY - 1 && j0 + TY * M < ny;
+  unsigned long long* const toCol =
+      inbox + ((size_t)(sendW ? b - 1 : sendE ? b + 1 : 0) * 4 + (sendW ? SIDE_E : SIDE_W)) * 64 + wave;
+  unsigned long long* const toS = inbox + ((size_t)(sendS ? b - tiles_x : 0) * 4 + SIDE_N) * 64 + li;
+  unsigned long long* const toN = inbox + ((size_t)(sendN ? b + tiles_x : 0) * 4 + SIDE_S) * 64 + li;
+  unsigned long long* const part = (unsigned long long*)(KA.res + kResPart);
+  unsigned long long* const bcast = (unsigned long long*)(KA.res + kResBcast);
+  unsigned long long* const line = bcast + 16 * (b & (kCopies - 1));
+  unsigned seq = sh.seq0;
+  double pq = 0.0, alpha = 0.0, rho_prev = rho, rnorm2 = st.rnorm2;
+  bool dead = false;
+  int n = 0;
+  while (true) {
+    unsigned long long* const pb = part + (n & 1) * 3 * kResMaxBlk;
+    // P: d = M r (first iteration) or d beta + M r, in registers and LDS.
+    const bool first = (it == 0);
+    if (tid_flat() == 0) sh.tiny[(n + 1) & 1] = 0;
+    bool tiny = false;
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const double z = wv[m] * rv[m];
+      double d = first ? z : dv[m] * beta + z;
+      if (!full) d = in[m] ? d : 0.0;
+      dv[m] = d;
+      lD[c0 + TY * m * P] = d;
+      tiny = tiny || (fabs(d) < kTinyD && d != 0.0);
+    }
+    if (multi && side >= 0 && side < 4) {
+      if (n > 0) {
+        unsigned long long* const w = mine + ((n - 1) & 1) * inbuf;
+        const long long t0 = wall_clock64();
+        unsigned long long x;
+        while (true) {
+          x = ring ? dev_load(w) : 0ull;
+          if (!__any(x == kSent)) break;
+          if (wall_clock64() - t0 > kWaitTicks) {
+            if (li == 0) sh.dead = 1;
+            break;
+          }
+        }
+        if (ring) dev_store(w, kSent);
+        rr = __longlong_as_double((long long)x);
+      }
+      const double z = rw * rr;
+      rd = first ? z : rd * beta + z;
+      if (ring) lD[ro] = rd;
+      tiny = tiny || (ring && fabs(rd) < kTinyD && rd != 0.0);
+    }
+    if (__any(tiny) && li == 0) sh.tiny[n & 1] = 1;
+    __syncthreads();
+    // q = A d. Differences of the region's d are zero or at least 2^-352 in
+    // magnitude where no d is a tiny number, and so are what div_fast divides
+    // after them; a numerator above its range gives a q that is not finite. A
+    // region with a tiny d, or a thread with such a q, divides.
+    bool slow = !fast || sh.tiny[n & 1] != 0;
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const int o = TY * m * P;
+      const double c = dv[m];
+      const double tx = div_fast(lD[oE + o] - c, dx) - div_fast(c - lD[oW + o], dx);
+      const double ty = div_fast(lD[oN[m]] - c, dy) - div_fast(c - lD[oS[m]], dy);
+      qv[m] = ((0.0 + div_fast(tx, dx)) + div_fast(ty, dy)) * sign;
+      slow = slow || !(fabs(qv[m]) < 0x1p900);
+    }
+    if (__any(slow)) {
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        const int o = TY * m * P;
+        const double q = lap_coherent5<double>(dv[m], lD[oE + o], lD[oW + o], lD[oN[m]], lD[oS[m]], nx, ny,
+                                               j0 + TY * m + wave, i, dx.b, dy.b) * sign;
+        qv[m] = slow ? q : qv[m];
+      }
+    }
+    if (any_id) {
+#pragma unroll
+      for (int m = 0; m < M; ++m)
+        if ((idm >> m) & 1u) qv[m] = dv[m];
+    }
+    double s0 = 0.0;
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      if (!full) qv[m] = in[m] ? qv[m] : 0.0;
+      s0 += dv[m] * qv[m];
+    }
+    s0 = wave_reduce<false>(s0);
+    if (li == 63) sh.wsum[0][wave] = s0;
+    __syncthreads();
+    if (!multi) {
+      pq = 0.0 + fold_waves(sh.wsum[0]);
+      alpha = rho / pq;
+    } else {
+      if (wave == 0) {
+        const double t = fold_waves(sh.wsum[0]);
+        if (li == 0) dev_store_f64(pb + b, t);
+        bool ok = true;
+        if (b == 0) {
+          double v[4];
+          ok = words_take(pb, li, nblk, v);
+          pq = fold_words(li, nblk, v);
+          alpha = rho / pq;
+          const long long u = __double_as_longlong(alpha);
+          const unsigned pay = (li & 1) ? (unsigned)(u >> 32) : (unsigned)u;
+          drain_vmem();
+          if (li < 2 * kCopies) dev_store(bcast + 16 * (li >> 1) + (li & 1), pay | ((unsigned long long)(seq + 1) << 32));
+        } else {
+          unsigned pay;
+          ok = bcast_wait(line, li, 2, seq + 1, pay);
+          const unsigned lo = __builtin_amdgcn_readlane(pay, 0), hi = __builtin_amdgcn_readlane(pay, 1);
+          alpha = __longlong_as_double((long long)((unsigned long long)lo | ((unsigned long long)hi << 32)));
+        }
+        if (li == 0) {
+          sh.val[0] = alpha;
+          if (!ok) sh.dead = 1;
+        }
+      }
+      seq += 1;
+      __syncthreads();
+      alpha = sh.val[0];
+      if (sh.dead) {
+        dead = true;
+        break;
+      }
+    }
+    // Q: x += alpha d, r -= alpha q, partials r.(M r) and r.r; the region's
+    // edges of r go to the neighbours' inboxes.
+    double s1 = 0.0, s2 = 0.0;
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      xv[m] = xv[m] + alpha * dv[m];
+      double r = rv[m] - alpha * qv[m];
+      if (!full) r = in[m] ? r : 0.0;
+      rv[m] = r;
+      const double z = wv[m] * r;
+      s1 += r * z;
+      s2 += r * r;
+    }
+    if (multi) {
+      const size_t ob = (size_t)(n & 1) * inbuf;
+      if (sendW || sendE) {
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+          if (in[m]) dev_store_f64(toCol + ob + TY * m, rv[m]);
+      }
+      if (sendS && in[0]) dev_store_f64(toS + ob, rv[0]);
+      if (sendN && in[M - 1]) dev_store_f64(toN + ob, rv[M - 1]);
+    }
+    s1 = wave_reduce<false>(s1);
+    s2 = wave_reduce<false>(s2);
+    if (li == 63) {
+      sh.wsum[1][wave] = s1;
+      sh.wsum[2][wave] = s2;
+    }
+    __syncthreads();
+    bool more = false;
+    n += 1;
+    it += 1;
+    it_total += 1;
+    if (!multi) {
+      rho_prev = rho;
+      rho = 0.0 + fold_waves(sh.wsum[1]);
+      rnorm2 = 0.0 + fold_waves(sh.wsum[2]);
+      beta = rho / rho_prev;
+      more = it_total < maxiter && !(sqrt(rnorm2) < atol) && !isnan(rnorm2) && n < kResIters;
+    } else {
+      if (wave == 0) {
+        const double t1 = fold_waves(sh.wsum[1]), t2 = fold_waves(sh.wsum[2]);
+        if (li < 2) dev_store_f64(pb + (1 + li) * kResMaxBlk + b, li ? t2 : t1);
+        bool ok = true;
+        if (b == 0) {
+          double v[4], w[4];
+          ok = words_take(pb + kResMaxBlk, li, nblk, v);
+          ok = words_take(pb + 2 * kResMaxBlk, li, nblk, w) && ok;
+          rho_prev = rho;
+          rho = fold_words(li, nblk, v);
+          rnorm2 = fold_words(li, nblk, w);
+          beta = rho / rho_prev;
+          more = it_total < maxiter && !(sqrt(rnorm2) < atol) && !isnan(rnorm2) && n < kResIters;
+          const long long u = __double_as_longlong(beta);
+          const int wd = li & 3;
+          const unsigned pay = wd == 0 ? (unsigned)u : wd == 1 ? (unsigned)(u >> 32) : (more ? 1u : 0u);
+          drain_vmem();
+          if (li < 4 * kCopies && wd < 3)
+            dev_store(bcast + 16 * (li >> 2) + wd, pay | ((unsigned long long)(seq + 1) << 32));
+        } else {
+          unsigned pay;
+          ok = bcast_wait(line, li, 3, seq + 1, pay);
+          const unsigned lo = __builtin_amdgcn_readlane(pay, 0), hi = __builtin_amdgcn_readlane(pay, 1);
+          beta = __longlong_as_double((long long)((unsigned long long)lo | ((unsigned long long)hi << 32)));
+          more = __builtin_amdgcn_readlane(pay, 2) != 0;
+        }
+        if (li == 0) {
+          sh.val[1] = beta;
+          sh.go = more ? 1 : 0;
+          if (!ok) sh.dead = 1;
+        }
+      }
+      seq += 1;
+      __syncthreads();
+      beta = sh.val[1];
+      more = sh.go != 0;
+      if (sh.dead) {
+        dead = true;
+        break;
+      }
+    }
+    if (!more) break;
+  }
+  if (dead) {
+    if (tid_flat() == 0) __hip_atomic_store(KA.active + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  }
+  // Leave the vectors and the state as a Q round and its tail leave them.
+  double* Dn = ((it - 1) & 1) ? D1 : D0;  // the last P's direction array
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    if (in[m]) {
+      const size_t k = (size_t)(j0 + TY * m + wave) * nx + i;
+      X[k] = xv[m];
+      R[k] = rv[m];
+      Dn[k] = dv[m];
+    }
+  }
+  if (multi && side >= 0 && side < 4) {  // the last Q's edges, which no P reads
+    unsigned long long* const w = mine + ((n - 1) & 1) * inbuf;
+    const long long t0 = wall_clock64();
+    while (true) {
+      const unsigned long long x = ring ? dev_load(w) : 0ull;
+      if (!__any(x == kSent) || wall_clock64() - t0 > kWaitTicks) break;
+    }
+    if (ring) dev_store(w, kSent);
+  }
+  if (b == 0 && tid_flat() == 0) {
+    st.it_run += it_total - st.it_total;
+    st.it = it;
+    st.it_total = it_total;
+    st.pq = pq;
+    st.alpha = alpha;
+    st.rho_prev = rho_prev;
+    st.rho = rho;
+    st.rnorm2 = rnorm2;
+    st.beta = beta;
+    st.pending = PH_IDLE;
+    cg_next(C, st);
+  }
+}
+
+}  // namespace pf

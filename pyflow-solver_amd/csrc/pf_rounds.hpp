@@ -106,6 +106,8 @@ struct PfCav {
   int ca;  // MIXED s-step rounds: 0 one PCG iteration per round; 1 two (4-cell halo); 2 three (6-cell halo)
   float cxf, cyf, invdf;  // (float)(1/dx^2), (float)(1/dy^2), (float)invd, formed on the host
   double lid, dx, dy, nu, cfl, growth, tol, invd, inner_rtol;
+  double rdx, rdy;  // RN(1/dx), RN(1/dy)
+  int fastdiv;      // FP64: dx and dy are divisors that div_fast divides by exactly (divisor_exact)
   void *u, *v, *p, *us, *vs, *r, *d0, *d1, *x;  // element type T
   void* r1;                                     // MIXED: r double-buffered (r, r1); p in d0/d1
   double *b, *x64;                              // x64 aliases x in FP64 mode
@@ -2174,7 +2176,8 @@ struct KArgs {
   int max_cav;
   int parity;
   int slot0;   // SINGLE: the cavity's slot
-  int pad;
+  int meet_ticks;  // resident solves: how long workgroups wait for each other to start (100 MHz clock)
+  char* res;   // exchange buffers of the resident solves (pf_resident.hpp); nullptr: one phase per launch
   PfCav cav0;  // SINGLE: the cavity's descriptor
 };
 
@@ -2364,11 +2367,16 @@ __device__ __attribute__((noinline)) void local_cg(const PfCav* __restrict__ Cg,
   if (tid < 2) part_out[(size_t)tid * nblk] = raw[tid];
 }
 
+}  // namespace pf
+#include "pf_resident.hpp"
+namespace pf {
+
 // Body of one round for workgroup b of cavity c. M > 0 (float32 only): the
 // cavity's region height in tiles. (Issuing the PCG region loads at entry,
 // before the phase is known, gained no time and gave wrong results in
 // batches with more workgroups than CUs; they are issued in the PCG branch.)
-template <class T, int U, int M, bool XD, bool MULTI>
+// RES (FP64): a P phase may run its whole solve in this launch (resident_cg64).
+template <class T, int U, int M, bool XD, bool MULTI, bool RES = false>
 __device__ __attribute__((always_inline)) inline void round_body(const KArgs& KA, const PfCav& C, const PfCav* Cg, int c, int b, PfScal& st,
                                   double (*sm)[NPS], double* tot, float* lds) {
   const int parity = KA.parity;
@@ -2486,7 +2494,23 @@ __device__ __attribute__((always_inline)) inline void round_body(const KArgs& KA
       }
     }
     block_partials_k<(XD ? KXD : 3), 0u>(acc, sm, part_out, nblk);
-  } else if (M == 0 && sizeof(T) == sizeof(double) && phase == PH_P && C.local && !isnan(st.rnorm2)) {
+  } else if (RES && phase == PH_P && !isnan(st.rnorm2) && resident_enter(KA, C, b, (ResShared*)sm)) {
+    if constexpr (RES) {
+      double* ld = (double*)lds;
+      switch (C.tpb) {
+        case 1: resident_cg64<1>(KA, C, st, sm, ld, b); break;
+        case 2: resident_cg64<2>(KA, C, st, sm, ld, b); break;
+        default: resident_cg64<4>(KA, C, st, sm, ld, b); break;
+      }
+    }
+    if (b == 0) {
+      __syncthreads();
+      if (tid == 0 && !st.dsetup) st.rounds_run += 1;
+      __syncthreads();
+      if (tid < NW32) dst[tid] = ((const uint32_t*)&st)[tid];
+    }
+    return;
+  } else if (!RES && M == 0 && sizeof(T) == sizeof(double) && phase == PH_P && C.local && !isnan(st.rnorm2)) {
     if constexpr (sizeof(T) == sizeof(double)) {
       if (C.tiles_y <= 4)
         local_cg<T, 4>(Cg, st, sm, tot, (double*)lds, part_out);
@@ -2830,6 +2854,21 @@ __global__ __launch_bounds__(NTH) void k_round(const KArgs KA) {
   } else {
     round_body<T, U, 0, false, MULTI>(KA, C, Cg, c, b, st, sm, tot, lds_dyn);
   }
+}
+
+// Single FP64 cavities whose workgroups all fit on the GPU at once: the rounds
+// of k_round, with each CG solve run by resident workgroups (pf_resident.hpp).
+__global__ __launch_bounds__(NTH) void k_round_res64(const KArgs KA) {
+  __shared__ PfScal st;
+  __shared__ double sm[NWAVE][NPS];
+  __shared__ double tot[NPS];
+  extern __shared__ float lds_dyn[];  // res64_lds_doubles(tpb) doubles
+  const PfCav& C = KA.cav0;
+  const PfCav* Cg = KA.cavs + KA.slot0;
+  const int lg = blockIdx.x - C.blk0;
+  const int b = ((C.blk0 & 7) == 0 && (C.nblk & 7) == 0) ? (lg & 7) * (C.nblk >> 3) + (lg >> 3) : lg;
+  if (b == 0 && tid_flat() == 0) resident_clear_meet(KA);
+  round_body<double, 2, 0, false, false, true>(KA, C, Cg, KA.slot0, b, st, sm, tot, lds_dyn);
 }
 
 // Batches whose cavities all run three PCG iterations per round (PfCav::ca
