@@ -89,7 +89,7 @@ struct pf_batch {
   int xd_kinds = 0;      // rounds of those cavities: bit 0 one PCG iteration, bit 1 two
   bool multi = false;    // some cavity has several regions per workgroup
   bool occ2 = false;     // every cavity fits the two-workgroups-per-CU kernel
-  int res_kind = 0;      // rounds with resident solves: 0 none, 1 FP64 (k_round_res64)
+  int res_kind = 0;      // rounds with resident solves: 0 none, 1 FP64 (k_round_res64), 2 MIXED (k_round_res32)
   char* dres = nullptr;  // their exchange buffers (KArgs::res), allocated when first used
   size_t dres_bytes = 0;
   bool res_ready = false;  // dres holds its resting values
@@ -330,16 +330,17 @@ static bool same_operator(const PfCav& a, const PfCav& b) { return a.op == b.op 
 
 static void drop_graphs(pf_batch* b);
 
-// Batches whose rounds may run a solve by resident workgroups: one FP64
-// cavity with one region of at most 4 tiles per workgroup and no more
+// Batches whose rounds may run a solve by resident workgroups: one cavity
+// (FP64, or MIXED with an FP32 iterate and two PCG iterations per round) with one region of at most 4 tiles per workgroup and no more
 // workgroups than CUs, so that all of them can be on the GPU at once
 // (PYFLOW_RESIDENT=0: never). Results are bitwise the same either way.
 static int resident_kind(const pf_batch* b) {
   if (b->single_slot < 0 || env_switch("PYFLOW_RESIDENT", 1) == 0) return 0;
   const PfCav& c = b->hcav[b->single_slot];
   if (c.rpw != 1 || c.tpb > 4 || c.nblk > std::min(b->num_cu, kResMaxBlk)) return 0;
-  if (c.nblk == 1 && !c.local) return 0;  // PYFLOW_LOCAL=0: one phase per launch
-  return b->prec == PF_PREC_FP64 ? 1 : 0;
+  if (b->prec == PF_PREC_FP64 && c.nblk == 1 && !c.local) return 0;  // PYFLOW_LOCAL=0: one phase per launch
+  if (b->prec == PF_PREC_FP64) return 1;
+  return c.ca == 1 && !c.xd ? 2 : 0;
 }
 
 // Runs (pf_batch_run, pf_batch_launch) let a launch run a whole solve; served
@@ -350,6 +351,16 @@ static int set_resident(pf_batch* b, bool on) {
   on = on && b->res_kind != 0;
   if (on != b->res_on) drop_graphs(b);  // their nodes carry KArgs::res
   if (on && (!b->res_on || !b->res_ready)) {
+    const PfCav& c = b->hcav[b->single_slot];
+    const size_t need = b->res_kind == 1 ? res64_bytes(c.nblk) : res32_bytes((size_t)c.nx * c.ny);
+    if (b->dres_bytes < need) {
+      if (b->dres) HIPCHK(hipFree(b->dres));
+      b->dres = nullptr;
+      b->dres_bytes = 0;
+      drop_graphs(b);
+      HIPCHK(hipMalloc((void**)&b->dres, need));
+      b->dres_bytes = need;
+    }
     HIPCHK(hipMemsetAsync(b->dres, 0xff, b->dres_bytes, b->stream));
     HIPCHK(hipMemsetAsync(b->dres + kResMeet, 0, 256, b->stream));
     b->res_ready = true;
@@ -403,16 +414,6 @@ static int sync_tables(pf_batch* b) {
     }
   b->res_kind = resident_kind(b);
   b->res_ready = false;
-  if (b->res_kind) {
-    const size_t need = res64_bytes(b->hcav[b->single_slot].nblk);
-    if (b->dres_bytes < need) {
-      if (b->dres) HIPCHK(hipFree(b->dres));
-      b->dres = nullptr;
-      b->dres_bytes = 0;
-      HIPCHK(hipMalloc((void**)&b->dres, need));
-      b->dres_bytes = need;
-    }
-  }
   HIPCHK(hipMemcpyAsync(b->dcav, b->hcav.data(), sizeof(PfCav) * b->max_cav, hipMemcpyHostToDevice, b->stream));
   if (!tiles.empty())
     HIPCHK(hipMemcpyAsync(b->dtile, tiles.data(), sizeof(int) * tiles.size(), hipMemcpyHostToDevice, b->stream));
@@ -489,16 +490,20 @@ static RoundLaunch round_launch(const pf_batch* b) {
       const bool one = b->single_slot >= 0;
       L.fn = b->multi ? (one ? (const void*)k_round_ca3<true, true> : (const void*)k_round_ca3<false, true>)
                       : (one ? (const void*)k_round_ca3<true, false> : (const void*)k_round_ca3<false, false>);
-    } else if (b->occ2)
+    } else if (b->res_kind == 2 && b->res_on)
+      L.fn = (const void*)k_round_res32;
+    else if (b->occ2)
       L.fn = b->single_slot >= 0 ? (const void*)k_round_occ2<true> : (const void*)k_round_occ2<false>;
     else
       L.fn = round_fn_u<float, 2>(b);  // U only shapes the FP64 P/Q loops
     L.lds = (size_t)b->lds_floats * sizeof(float);
+    if (b->res_kind == 2 && b->res_on)
+      L.lds = std::max(L.lds, res32_lds_floats(b->hcav[b->single_slot].tpb) * sizeof(float));
   } else {
     L.fn = b->unroll >= 4 ? round_fn_u<double, 4>(b) : b->unroll == 2 ? round_fn_u<double, 2>(b)
                                                                       : round_fn_u<double, 1>(b);
     L.lds = (size_t)b->lds_floats * sizeof(float);
-    if (b->res_kind == 1) {
+    if (b->res_kind == 1 && b->res_on) {
       L.fn = (const void*)k_round_res64;
       L.lds = std::max(L.lds, res64_lds_doubles(b->hcav[b->single_slot].tpb) * sizeof(double));
     }
@@ -814,8 +819,9 @@ int pf_batch_workspace_bytes(int precision, int ncav, const pf_cavity_params* pa
 static int graph_len_of(int rounds) { return rounds <= 0 ? 0 : std::min(1024, std::max(2, rounds & ~1)); }
 
 static int allow_region_lds() {
-  const int bytes = std::max({region_lds_floats(8), ca_lds_floats(4), ca3_lds_floats(4)}) * (int)sizeof(float);
-  const void* fns[16] = {
+  const int bytes = std::max({region_lds_floats(8), ca_lds_floats(4), ca3_lds_floats(4), res32_lds_floats(4)}) * (int)sizeof(float);
+  const void* fns[17] = {
+      (const void*)k_round_res32,
       (const void*)k_round_ca3<true, false>, (const void*)k_round_ca3<false, false>,
       (const void*)k_round_ca3<true, true>, (const void*)k_round_ca3<false, true>,
       (const void*)k_round_occ2<true>, (const void*)k_round_occ2<false>,

@@ -24,8 +24,12 @@
 //                 written again;
 //   tail results  words of 32 bits of payload and a 32-bit sequence number,
 //                 stored by workgroup 0 on kCopies lines (fewer readers per line);
-//   region edges  one inbox per region side, read by that region only, which
-//                 puts kSent back; two buffers alternate here too.
+//   region edges  FP64: one inbox per region side, read by that region only,
+//                 which puts kSent back; two buffers alternate here too.
+//                 MIXED: a region's outer four rows and columns of (r, p), at
+//                 their place in the grid, followed by the region's sequence
+//                 number once the stores have completed; its neighbours wait
+//                 for that number. Two buffers alternate.
 // A sum or cell that equals kSent (a NaN) is stored as another NaN.
 #pragma once
 
@@ -43,9 +47,11 @@ constexpr unsigned kMeetAbort = 0x10000u;
 // Layout of KArgs::res (bytes; every block starts on a 128-byte line).
 constexpr size_t kResMeet = 0;             // arrival words, one per round parity, 128 bytes apart
 constexpr size_t kResBcast = 512;          // kCopies lines of 16 words
-constexpr size_t kResPart = 4096;          // 2 x 3 x kResMaxBlk words
-constexpr size_t kResInbox = kResPart + 2 * 3 * kResMaxBlk * 8;  // [2][nblk][4 sides][64] words
-__host__ __device__ constexpr size_t res64_bytes(int nblk) { return kResInbox + (size_t)2 * nblk * 4 * 64 * 8; }
+constexpr size_t kResPart = 4096;          // FP64: 2 x 3 x kResMaxBlk words; MIXED: 2 x kResMaxBlk lines of 16 words
+constexpr size_t kResFlag = kResPart + 2 * kResMaxBlk * 128;  // MIXED: a sequence number per workgroup, 128 bytes apart
+constexpr size_t kResData = kResFlag + kResMaxBlk * 128;      // FP64: inboxes [2][nblk][4 sides][64]; MIXED: (r, p) [2][ny][nx]
+__host__ __device__ constexpr size_t res64_bytes(int nblk) { return kResData + (size_t)2 * nblk * 4 * 64 * 8; }
+__host__ __device__ constexpr size_t res32_bytes(size_t cells) { return kResData + 2 * cells * 8; }
 enum { SIDE_W = 0, SIDE_E = 1, SIDE_S = 2, SIDE_N = 3 };
 
 constexpr int kResPitch = TX + 3;  // LDS pitch of the FP64 direction: 64 columns, a ring, odd
@@ -64,26 +70,25 @@ __device__ inline void dev_store_f64(unsigned long long* p, double v) {
 // Every memory operation of this wave has completed.
 __device__ inline void drain_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// Words the workgroup shares during a resident solve; they overlay the
-// reduction array, which the solve does not use.
+// Words a workgroup shares during a resident solve.
 struct ResShared {
-  double val[4];        // alpha, or beta
+  double val[2];          // FP64: alpha, beta
+  float coef[4];          // MIXED: alpha_k, beta_k, alpha_k+1, beta_k+1
   double wsum[3][NWAVE];  // wave totals: P, and the two of Q
   unsigned seq0;        // sequence number of the last broadcast before this launch
   int go, dead;
   int tiny[2];  // some d of the region or its ring is a tiny number, by iteration parity
 };
-static_assert(sizeof(ResShared) <= sizeof(double) * NWAVE * NPS, "ResShared overlays the reduction array");
 
 // Whether this launch's workgroups are all running (see above). Every thread
 // of every workgroup of the cavity calls it once per launch at most.
 __device__ inline bool resident_enter(const KArgs& KA, const PfCav& C, int b, ResShared* sh) {
   if (KA.res == nullptr) return false;
   const int nblk = C.nblk;
-  __syncthreads();  // the preamble's use of the overlaid array has ended
   if (tid_flat() == 0) {
     sh->dead = 0;
     sh->go = 1;
+    sh->seq0 = 0;
     sh->tiny[0] = sh->tiny[1] = 0;
     if (nblk > 1) {
       unsigned* meet = (unsigned*)(KA.res + kResMeet + 128 * KA.parity);
@@ -201,8 +206,7 @@ __device__ inline double fold_waves(const double* w) {
 // tails' scalars from the wave totals.
 template <int M>
 __device__ __attribute__((always_inline)) inline void resident_cg64(const KArgs& KA, const PfCav& C, PfScal& st,
-                                                                    double (*sm)[NPS], double* __restrict__ lD, int b) {
-  ResShared& sh = *(ResShared*)sm;
+                                                                    ResShared& sh, double* __restrict__ lD, int b) {
   constexpr int P = kResPitch;
   const int nx = C.nx, ny = C.ny, nblk = C.nblk, tiles_x = C.tiles_x;
   const int li = threadIdx.x;
@@ -258,7 +262,7 @@ __device__ __attribute__((always_inline)) inline void resident_cg64(const KArgs&
   bool ring = false;
   double rr = 0.0, rd = 0.0, rw = 0.0;
   int ro = 0;
-  unsigned long long* inbox = (unsigned long long*)(KA.res + kResInbox);
+  unsigned long long* inbox = (unsigned long long*)(KA.res + kResData);
   unsigned long long* mine = inbox;
   if (multi && side >= 0 && side < 4) {
     int gi, gj, row, col;
@@ -530,6 +534,396 @@ __device__ __attribute__((always_inline)) inline void resident_cg64(const KArgs&
     st.beta = beta;
     st.pending = PH_IDLE;
     cg_next(C, st);
+  }
+}
+
+constexpr int kGatherPitch = kResMaxBlk + 1;
+// LDS of resident_ca: p, z = M r and M A p on a region with its 4-cell frame,
+// and the sums that workgroup 0 collects.
+__host__ __device__ constexpr int res32_lds_floats(int m) {
+  return (3 * (TY * m + 8) * HQ + 1) / 2 * 2 + 2 * KCA * kGatherPitch;
+}
+
+// The two-iteration PCG rounds of an inner solve of a MIXED cavity (region_ca
+// and tail_ca, FP32 iterate), from a round that runs iterations to the round
+// that ends the inner solve or kResIters rounds. A thread keeps r, p, x of its M
+// cells, and with them a = A p, c = A M a and e = A z: the round forms them of
+// the new basis for its Gram sums, and the next round needs the same values
+// again, so it evaluates three stencils per cell instead of six. p, z and M a
+// lie in LDS with the frame. Of the frame, a region computes distances 1 and 2
+// itself (r, p and a by their owner's expressions) and receives distances 3 and
+// 4 from its neighbours after every round. All that does not depend on the new
+// step lengths (receiving the frame; a at distances 2 and 3; c and e at
+// distances 1 and 2) runs while the sums are under way. Cell expressions, sums,
+// reduction, fold and tail are those of region_ca's rounds in their order, so the
+// results are the same bits. A missing neighbour at the domain's edge is read
+// as the cell itself (its difference is +0, as region_ca's ghost copies make it).
+template <int M>
+__device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& KA, const PfCav& C, PfScal& st,
+                                                                  double (*sm)[NPS], double* tot, ResShared& sh,
+                                                                  float* __restrict__ lds, int b) {
+  constexpr int RH = TY * M, NR = RH + 8, TP = TY * HQ;
+  constexpr int F1 = ca_frame_cells(RH, 1), F2 = ca_frame_cells(RH, 2), F3 = ca_frame_cells(RH, 3);
+  constexpr int F4 = ca_frame_cells(RH, 4);
+  static_assert(F3 <= NTH && F4 <= NTH + 64, "a frame cell per thread, and one more in wave 0");
+  float* __restrict__ lP = lds;
+  float* __restrict__ lZ = lds + NR * HQ;
+  float* __restrict__ lMA = lds + 2 * NR * HQ;
+  double* __restrict__ lG = (double*)(lds + (3 * NR * HQ + 1) / 2 * 2);  // [KCA][kGatherPitch]
+  const int nx = C.nx, ny = C.ny, nblk = C.nblk, tiles_x = C.tiles_x;
+  const int li = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const int tid = wave * TX + li;
+  const int rx = b % tiles_x, ry = b / tiles_x;
+  const int i0 = rx * TX, j0 = ry * RH;
+  const int i = i0 + li;
+  const bool full = (i0 + TX <= nx) && (j0 + RH <= ny);
+  const bool pinned = (C.op == 0);
+  const float scx = pinned ? -C.cxf : C.cxf, scy = pinned ? -C.cyf : C.cyf;
+  auto minv = [&](int j, int ii) -> float {
+    if (!C.jacobi) return 1.0f;
+    return (ii == 0 || ii == nx - 1 || j == 0 || j == ny - 1) ? 1.0f : C.invdf;
+  };
+  auto ident = [&](int j, int ii) -> bool {
+    return pinned ? (j == 0 && ii == 0) : (j == 0 || j == ny - 1 || ii == 0 || ii == nx - 1);
+  };
+  auto lap = [&](const float* L, int o, int oe, int ow, int on, int os) -> float {
+    const float c = L[o];
+    return __fmul_rn((L[oe] - c) - (c - L[ow]), scx) + __fmul_rn((L[on] - c) - (c - L[os]), scy);
+  };
+  const size_t n2 = (size_t)nx * ny;
+  const float* __restrict__ R = mixed_r(C, KA.parity);
+  const float* __restrict__ Pold = mixed_p(C, KA.parity ^ 1);
+  float* __restrict__ X = (float*)C.x;
+  unsigned long long* const xch = (unsigned long long*)(KA.res + kResData);
+
+  // Own cells.
+  const int o0 = (wave + 4) * HQ + li + 4;
+  const int oE = o0 + ((i + 1 < nx) ? 1 : 0), oW = o0 - ((i > 0) ? 1 : 0);
+  int oN[M], oS[M];
+  float ro[M], po[M], xo[M], ao[M], cv[M], ev[M], mo[M];
+  unsigned inm = 0, idm = 0, pub = 0;  // in the domain; identity row; to be published (bit m)
+  const bool pubcol = (li < 4 && rx > 0) || (li >= TX - 4 && i0 + TX < nx);
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    const int row = TY * m + wave, j = j0 + row;
+    const bool in = (i < nx) && (j < ny);
+    const size_t k = in ? (size_t)j * nx + i : 0;
+    ro[m] = R[k];
+    po[m] = Pold[k];
+    xo[m] = X[k];
+    mo[m] = minv(j, i);
+    oN[m] = o0 + m * TP + ((j + 1 < ny) ? HQ : 0);
+    oS[m] = o0 + m * TP - ((j > 0) ? HQ : 0);
+    if (in) {
+      inm |= 1u << m;
+      if (ident(j, i)) idm |= 1u << m;
+      if (pubcol || (row < 4 && j0 > 0) || (row >= RH - 4 && j0 + RH < ny)) pub |= 1u << m;
+    }
+  }
+  const bool any_id = __any(idm != 0);
+  // Frame cells: q0 per thread, counted down so that wave 0, which also waits
+  // for the broadcasts, has the outermost; q1 in wave 0 where the frame has more
+  // than NTH cells.
+  const int q0 = NTH - 1 - tid;
+  int fo = 0, fE = 0, fW = 0, fN = 0, fS = 0;
+  bool fin = false, fid = false;
+  float fr = 0.f, fp = 0.f, fa = 0.f, fc = 0.f, fe = 0.f, fm = 0.f;
+  size_t fk = 0;
+  if (q0 < F4) {
+    int row, col;
+    ca_frame_cell(RH, q0, row, col);
+    const int gj = j0 + row - 4, gi = i0 + col - 4;
+    fin = gi >= 0 && gi < nx && gj >= 0 && gj < ny;
+    if (fin) {
+      fo = row * HQ + col;
+      fE = fo + ((gi + 1 < nx) ? 1 : 0);
+      fW = fo - ((gi > 0) ? 1 : 0);
+      fN = fo + ((gj + 1 < ny) ? HQ : 0);
+      fS = fo - ((gj > 0) ? HQ : 0);
+      fid = ident(gj, gi);
+      fm = minv(gj, gi);
+      fk = (size_t)gj * nx + gi;
+      fr = R[fk];
+      fp = Pold[fk];
+    }
+  }
+  const bool fin1 = fin && q0 < F1, fin2 = fin && q0 < F2, fin3 = fin && q0 < F3, finX = fin && q0 >= F2;
+  int go1 = 0;  // q1: LDS word and grid cell
+  bool gin = false;
+  float gm = 0.f, gr = 0.f, gp = 0.f;
+  size_t gk = 0;
+  if (F4 > NTH && NTH + tid < F4) {
+    int row, col;
+    ca_frame_cell(RH, NTH + tid, row, col);
+    const int gj = j0 + row - 4, gi = i0 + col - 4;
+    gin = gi >= 0 && gi < nx && gj >= 0 && gj < ny;
+    if (gin) {
+      go1 = row * HQ + col;
+      gm = minv(gj, gi);
+      gk = (size_t)gj * nx + gi;
+      gr = R[gk];
+      gp = Pold[gk];
+    }
+  }
+  const bool loads = __any(finX || gin);  // this wave receives frame cells
+  // The neighbour whose sequence number lane 0..7 watches.
+  const unsigned long long* flag = nullptr;
+  unsigned long long* const flags = (unsigned long long*)(KA.res + kResFlag);
+  if (li < 8) {
+    const int t = li < 4 ? li : li + 1;  // 3 x 3 without the centre
+    const int ex = t % 3 - 1, ey = t / 3 - 1;
+    const int nxr = rx + ex, nyr = ry + ey;
+    if (nxr >= 0 && nxr < tiles_x && nyr >= 0 && nyr * RH < ny) flag = flags + (size_t)(nyr * tiles_x + nxr) * 16;
+  }
+  unsigned long long* const part = (unsigned long long*)(KA.res + kResPart);
+  unsigned long long* const bcast = (unsigned long long*)(KA.res + kResBcast);
+  unsigned long long* const line = bcast + 16 * (b & (kCopies - 1));
+  const unsigned seq0 = sh.seq0;
+
+  // The stencils of the first basis.
+  auto own_put = [&](float* L, const float (&v)[M]) {
+#pragma unroll
+    for (int m = 0; m < M; ++m) L[o0 + m * TP] = v[m];
+  };
+  {
+    float z[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) z[m] = mo[m] * ro[m];
+    own_put(lP, po);
+    own_put(lZ, z);
+  }
+  if (fin) {
+    lP[fo] = fp;
+    lZ[fo] = fm * fr;
+  }
+  if (gin) {
+    lP[go1] = gp;
+    lZ[go1] = gm * gr;
+  }
+  __syncthreads();
+  auto own_a = [&]() {  // a = A p, M a into LDS
+#pragma unroll
+    for (int m = 0; m < M; ++m) ao[m] = lap(lP, o0 + m * TP, oE + m * TP, oW + m * TP, oN[m], oS[m]);
+    if (any_id) {
+#pragma unroll
+      for (int m = 0; m < M; ++m)
+        if ((idm >> m) & 1u) ao[m] = po[m];
+    }
+#pragma unroll
+    for (int m = 0; m < M; ++m) lMA[o0 + m * TP] = mo[m] * ao[m];
+  };
+  auto own_ce = [&](int m) {  // c = A M a, e = A z
+    cv[m] = lap(lMA, o0 + m * TP, oE + m * TP, oW + m * TP, oN[m], oS[m]);
+    ev[m] = lap(lZ, o0 + m * TP, oE + m * TP, oW + m * TP, oN[m], oS[m]);
+    if (any_id && ((idm >> m) & 1u)) {
+      cv[m] = mo[m] * ao[m];
+      ev[m] = mo[m] * ro[m];
+    }
+  };
+  auto frame_a = [&]() {
+    const float v = lap(lP, fo, fE, fW, fN, fS);
+    fa = fid ? fp : v;
+    lMA[fo] = fm * fa;
+  };
+  auto frame_ce = [&]() {
+    const float v = lap(lMA, fo, fE, fW, fN, fS), w = lap(lZ, fo, fE, fW, fN, fS);
+    fc = fid ? fm * fa : v;
+    fe = fid ? fm * fr : w;
+  };
+  own_a();
+  if (fin3) frame_a();
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < M; ++m) own_ce(m);
+  if (fin2) frame_ce();
+  float a0 = (float)st.ca0, b0 = (float)st.cb0, a1 = (float)st.ca1, b1 = (float)st.cb1;
+  __syncthreads();
+  bool dead = false;
+  int n = 0;
+  while (true) {
+    const unsigned seq = seq0 + 1 + (unsigned)n;
+    // The two steps (ca_steps).
+    unsigned long long* const xb = xch + (n & 1) * n2;
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const float z = mo[m] * ro[m], ma = mo[m] * ao[m];
+      const float p1 = (z - a0 * ma) + b0 * po[m];
+      const float ap1 = (ev[m] - a0 * cv[m]) + b0 * ao[m];
+      const float r2 = (ro[m] - a0 * ao[m]) - a1 * ap1;
+      const float z2 = mo[m] * r2;
+      const float p2 = z2 + b1 * p1;
+      xo[m] = (xo[m] + a0 * po[m]) + a1 * p1;
+      ro[m] = r2;
+      po[m] = p2;
+      lP[o0 + m * TP] = p2;
+      lZ[o0 + m * TP] = z2;
+      if ((pub >> m) & 1u)
+        dev_store(xb + (size_t)(j0 + TY * m + wave) * nx + i,
+                  (unsigned long long)__float_as_uint(r2) | ((unsigned long long)__float_as_uint(p2) << 32));
+    }
+    if (fin2) {
+      const float z = fm * fr, ma = fm * fa;
+      const float p1 = (z - a0 * ma) + b0 * fp;
+      const float ap1 = (fe - a0 * fc) + b0 * fa;
+      fr = (fr - a0 * fa) - a1 * ap1;
+      const float z2 = fm * fr;
+      fp = z2 + b1 * p1;
+      lP[fo] = fp;
+      lZ[fo] = z2;
+    }
+    __syncthreads();
+    own_a();
+    if (fin1) frame_a();
+    __syncthreads();
+    // c, e and the Gram sums of the new basis (pass 5 of region_ca).
+    double acc[NP] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      own_ce(m);
+      if (full || ((inm >> m) & 1u)) {
+        const double p2 = po[m], z2 = mo[m] * ro[m], r2 = ro[m], a2 = ao[m];
+        const double ma2 = mo[m] * ao[m], c2 = cv[m], mc2 = mo[m] * cv[m], e2 = ev[m], me2 = mo[m] * ev[m];
+        acc[0] = __fma_rn(p2, a2, acc[0]);
+        acc[1] = __fma_rn(p2, c2, acc[1]);
+        acc[2] = __fma_rn(p2, e2, acc[2]);
+        acc[3] = __fma_rn(a2, ma2, acc[3]);
+        acc[4] = __fma_rn(a2, mc2, acc[4]);
+        acc[5] = __fma_rn(a2, z2, acc[5]);
+        acc[6] = __fma_rn(a2, me2, acc[6]);
+        acc[7] = __fma_rn(c2, mc2, acc[7]);
+        acc[8] = __fma_rn(c2, z2, acc[8]);
+        acc[9] = __fma_rn(c2, me2, acc[9]);
+        acc[10] = __fma_rn(r2, z2, acc[10]);
+        acc[11] = __fma_rn(z2, e2, acc[11]);
+        acc[12] = __fma_rn(e2, me2, acc[12]);
+        acc[13] = __fma_rn(r2, r2, acc[13]);
+      }
+    }
+    wave_partials_ca(acc, sm);
+    drain_vmem();  // the published cells are in memory before the barrier, so before the flag
+    __syncthreads();
+    unsigned long long* const pb = part + (size_t)(n & 1) * kResMaxBlk * 16;
+    if (tid < KCA) {
+      double t = sm[0][tid];
+#pragma unroll
+      for (int w = 1; w < NWAVE; ++w) t += sm[w][tid];
+      dev_store_f64(pb + 16 * b + tid, t);
+    }
+    if (tid == NTH - 1) dev_store(flags + 16 * b, (unsigned long long)seq);
+    // The frame at distances 3 and 4.
+    if (loads) {
+      const long long t0 = wall_clock64();
+      while (true) {
+        const unsigned f = flag ? (unsigned)dev_load(flag) : seq;
+        if (!__any((int)(f - seq) < 0)) break;
+        if (wall_clock64() - t0 > kWaitTicks) {
+          if (li == 0) sh.dead = 1;
+          break;
+        }
+      }
+      asm volatile("" ::: "memory");  // the frame is loaded after its flags were seen
+    }
+    unsigned long long fx = 0, gx = 0;
+    if (finX) fx = dev_load(xb + fk);
+    if (gin) gx = dev_load(xb + gk);
+    if (b == 0) {  // collect the sums
+      unsigned long long x[4];
+      const long long t0 = wall_clock64();
+      while (true) {
+        bool miss = false;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int w = tid + NTH * t;
+          x[t] = ((w >> 4) < nblk && (w & 15) < KCA) ? dev_load(pb + w) : 0ull;
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) miss |= x[t] == kSent;
+        if (!__any(miss)) break;
+        if (wall_clock64() - t0 > kWaitTicks) {
+          if (li == 0) sh.dead = 1;
+          break;
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int w = tid + NTH * t;
+        if ((w >> 4) < nblk && (w & 15) < KCA) {
+          lG[(w & 15) * kGatherPitch + (w >> 4)] = __longlong_as_double((long long)x[t]);
+          dev_store(pb + w, kSent);
+        }
+      }
+    }
+    if (finX) {
+      fr = __uint_as_float((unsigned)fx);
+      fp = __uint_as_float((unsigned)(fx >> 32));
+      lP[fo] = fp;
+      lZ[fo] = fm * fr;
+    }
+    if (gin) {
+      lP[go1] = __uint_as_float((unsigned)(gx >> 32));
+      lZ[go1] = gm * __uint_as_float((unsigned)gx);
+    }
+    __syncthreads();
+    if (b == 0 && wave < KCA) {
+      double v = 0.0;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (li + 64 * t < nblk) v = v + lG[wave * kGatherPitch + li + 64 * t];
+      v = wave_reduce<false>(v);
+      if (li == 63) tot[wave] = v;
+    }
+    if (fin3 && !fin1) frame_a();
+    __syncthreads();
+    if (wave == 0) {
+      bool ok = true;
+      if (b == 0) {
+        if (li == 63) {
+          tail_ca(C, st, tot);
+          sh.go = (st.phase == PH_CG && n + 1 < kResIters) ? 1 : 0;
+          sh.coef[0] = (float)st.ca0;
+          sh.coef[1] = (float)st.cb0;
+          sh.coef[2] = (float)st.ca1;
+          sh.coef[3] = (float)st.cb1;
+        }
+        const int wd = li & 7;
+        drain_vmem();  // the collected words are back at kSent
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // lane 63's results, within the wave
+        const unsigned pay = wd < 4 ? __float_as_uint(sh.coef[wd]) : (unsigned)sh.go;
+        if (wd < 5) dev_store(bcast + 16 * (li >> 3) + wd, pay | ((unsigned long long)seq << 32));
+      } else {
+        unsigned pay;
+        ok = bcast_wait(line, li, 5, seq, pay);
+        if (li < 4) sh.coef[li] = __uint_as_float(pay);
+        if (li == 4) sh.go = (int)pay;
+      }
+      if (!ok && li == 0) sh.dead = 1;
+    }
+    if (fin2) frame_ce();
+    n += 1;
+    __syncthreads();
+    a0 = sh.coef[0];
+    b0 = sh.coef[1];
+    a1 = sh.coef[2];
+    b1 = sh.coef[3];
+    dead = sh.dead != 0;
+    if (dead || sh.go == 0) break;
+  }
+  if (dead) {
+    if (tid == 0) __hip_atomic_store(KA.active + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  }
+  // Leave the vectors as a round of this parity leaves them.
+  float* __restrict__ Rn = mixed_r(C, KA.parity ^ 1);
+  float* __restrict__ Pn = mixed_p(C, KA.parity);
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    if ((inm >> m) & 1u) {
+      const size_t k = (size_t)(j0 + TY * m + wave) * nx + i;
+      Rn[k] = ro[m];
+      Pn[k] = po[m];
+      X[k] = xo[m];
+    }
   }
 }
 

@@ -2043,7 +2043,7 @@ __device__ __attribute__((always_inline)) inline double swap_sum(double x, doubl
   const double ys = __longlong_as_double((long long)((unsigned long long)lo[1] | ((unsigned long long)hi[1] << 32)));
   return xs + ys;
 }
-__device__ inline void block_partials_ca(double (&v)[NP], double (*sm)[NPS], double* dst, int stride) {
+__device__ __attribute__((always_inline)) inline void wave_partials_ca(double (&v)[NP], double (*sm)[NPS]) {
   static_assert(KCA <= 16 && NP >= 16, "16 slots carried through the exchange");
   const int tid = tid_flat();
   const int lane = tid & 63, wave = tid >> 6;
@@ -2078,6 +2078,10 @@ __device__ inline void block_partials_ca(double (&v)[NP], double (*sm)[NPS], dou
   d = d + dpp_full<0xB1>(d);  // quad_perm [1,0,3,2]
   const int q = lane >> 2;
   if ((lane & 3) == 0 && q < KCA) sm[wave][q] = d;
+}
+__device__ inline void block_partials_ca(double (&v)[NP], double (*sm)[NPS], double* dst, int stride) {
+  const int tid = tid_flat();
+  wave_partials_ca(v, sm);
   __syncthreads();
   if (tid < KCA) {
     double t = sm[0][tid];
@@ -2378,7 +2382,7 @@ namespace pf {
 // RES (FP64): a P phase may run its whole solve in this launch (resident_cg64).
 template <class T, int U, int M, bool XD, bool MULTI, bool RES = false>
 __device__ __attribute__((always_inline)) inline void round_body(const KArgs& KA, const PfCav& C, const PfCav* Cg, int c, int b, PfScal& st,
-                                  double (*sm)[NPS], double* tot, float* lds) {
+                                  double (*sm)[NPS], double* tot, float* lds, ResShared* rsh = nullptr) {
   const int parity = KA.parity;
   const int tid = tid_flat();
   const uint32_t* src = (const uint32_t*)(KA.scal + (size_t)(parity ^ 1) * KA.max_cav + c);
@@ -2494,13 +2498,13 @@ __device__ __attribute__((always_inline)) inline void round_body(const KArgs& KA
       }
     }
     block_partials_k<(XD ? KXD : 3), 0u>(acc, sm, part_out, nblk);
-  } else if (RES && phase == PH_P && !isnan(st.rnorm2) && resident_enter(KA, C, b, (ResShared*)sm)) {
+  } else if (RES && phase == PH_P && !isnan(st.rnorm2) && resident_enter(KA, C, b, rsh)) {
     if constexpr (RES) {
       double* ld = (double*)lds;
       switch (C.tpb) {
-        case 1: resident_cg64<1>(KA, C, st, sm, ld, b); break;
-        case 2: resident_cg64<2>(KA, C, st, sm, ld, b); break;
-        default: resident_cg64<4>(KA, C, st, sm, ld, b); break;
+        case 1: resident_cg64<1>(KA, C, st, *rsh, ld, b); break;
+        case 2: resident_cg64<2>(KA, C, st, *rsh, ld, b); break;
+        default: resident_cg64<4>(KA, C, st, *rsh, ld, b); break;
       }
     }
     if (b == 0) {
@@ -2558,10 +2562,12 @@ __device__ __attribute__((always_inline)) inline void round_body(const KArgs& KA
 // partials are folded by one wave per slot: wave w sums slot w of every
 // workgroup (per lane: increasing workgroup index; then the DPP tree), so all
 // fourteen slots of the PCG round fold in parallel; thread 63 runs the tail.
-template <int M, bool MULTI, bool XD, int V = 0>
+// RES: a round that runs iterations may run the rest of its inner solve in this
+// launch (resident_ca).
+template <int M, bool MULTI, bool XD, int V = 0, bool RES = false>
 __device__ __attribute__((always_inline)) inline void round_body_ca(const KArgs& KA, const PfCav& C, const PfCav* Cg, int c,
                                                                     int b, PfScal& st, double (*sm)[NPS], double* tot,
-                                                                    float* lds) {
+                                                                    float* lds, ResShared* rsh = nullptr) {
   const int parity = KA.parity;
   const int tid = tid_flat();
   const uint32_t* src = (const uint32_t*)(KA.scal + (size_t)(parity ^ 1) * KA.max_cav + c);
@@ -2619,6 +2625,18 @@ __device__ __attribute__((always_inline)) inline void round_body_ca(const KArgs&
       if (tid == 0 && newly_done) atomicSub(KA.active, 1);
     }
     return;
+  }
+  if constexpr (RES) {
+    if (phase == PH_CG && st.ca_inc > 0 && resident_enter(KA, C, b, rsh)) {
+      resident_ca<M>(KA, C, st, sm, tot, *rsh, lds, b);
+      if (b == 0) {
+        __syncthreads();
+        if (tid == 0 && !st.dsetup) st.rounds_run += 1;
+        __syncthreads();
+        if (tid < NW32) dst[tid] = ((const uint32_t*)&st)[tid];
+      }
+      return;
+    }
   }
   PhaseArgs A;
   A.dt = st.dt;
@@ -2862,13 +2880,34 @@ __global__ __launch_bounds__(NTH) void k_round_res64(const KArgs KA) {
   __shared__ PfScal st;
   __shared__ double sm[NWAVE][NPS];
   __shared__ double tot[NPS];
+  __shared__ ResShared rsh;
   extern __shared__ float lds_dyn[];  // res64_lds_doubles(tpb) doubles
   const PfCav& C = KA.cav0;
   const PfCav* Cg = KA.cavs + KA.slot0;
   const int lg = blockIdx.x - C.blk0;
   const int b = ((C.blk0 & 7) == 0 && (C.nblk & 7) == 0) ? (lg & 7) * (C.nblk >> 3) + (lg >> 3) : lg;
   if (b == 0 && tid_flat() == 0) resident_clear_meet(KA);
-  round_body<double, 2, 0, false, false, true>(KA, C, Cg, KA.slot0, b, st, sm, tot, lds_dyn);
+  round_body<double, 2, 0, false, false, true>(KA, C, Cg, KA.slot0, b, st, sm, tot, lds_dyn, &rsh);
+}
+
+// The same for single MIXED cavities with an FP32 iterate and two PCG
+// iterations per round.
+__global__ __launch_bounds__(NTH) void k_round_res32(const KArgs KA) {
+  __shared__ PfScal st;
+  __shared__ double sm[NWAVE][NPS];
+  __shared__ double tot[NPS];
+  __shared__ ResShared rsh;
+  extern __shared__ float lds_dyn[];  // ca_lds_floats(tpb) or res32_lds_floats(tpb) floats
+  const PfCav& C = KA.cav0;
+  const PfCav* Cg = KA.cavs + KA.slot0;
+  const int lg = blockIdx.x - C.blk0;
+  const int b = ((C.blk0 & 7) == 0 && (C.nblk & 7) == 0) ? (lg & 7) * (C.nblk >> 3) + (lg >> 3) : lg;
+  if (b == 0 && tid_flat() == 0) resident_clear_meet(KA);
+  switch (C.tpb) {
+    case 1: round_body_ca<1, false, false, 3, true>(KA, C, Cg, KA.slot0, b, st, sm, tot, lds_dyn, &rsh); break;
+    case 2: round_body_ca<2, false, false, 3, true>(KA, C, Cg, KA.slot0, b, st, sm, tot, lds_dyn, &rsh); break;
+    default: round_body_ca<4, false, false, 3, true>(KA, C, Cg, KA.slot0, b, st, sm, tot, lds_dyn, &rsh); break;
+  }
 }
 
 // Batches whose cavities all run three PCG iterations per round (PfCav::ca

@@ -110,8 +110,44 @@ def test_fp64_shapes_bitwise(nx, ny, rows, maxiter, jacobi):
         assert new[2] < ref[2]
 
 
-@pytest.mark.parametrize("nx,ny", [(100, 70), (64, 64)])
-def test_fp64_steps_bitwise(nx, ny):
+@pytest.mark.parametrize("nx,ny,rows,maxiter,op,jacobi", [
+    (2, 2, 0, 50, "pinned", True),
+    (5, 3, 0, 50, "dirichlet", True),
+    (64, 16, 1, 500, "pinned", True),      # one full region of one tile
+    (65, 17, 0, 800, "pinned", True),      # frames with one-cell neighbours
+    (67, 66, 4, 1500, "dirichlet", True),  # neighbours narrower than the frame
+    (2, 300, 0, 1500, "pinned", True),
+    (300, 3, 0, 1500, "pinned", False),
+    (130, 33, 1, 2000, "pinned", True),
+    (131, 97, 2, 2000, "pinned", True),
+    (192, 128, 4, 3000, "pinned", False),
+    (256, 192, 4, 3000, "dirichlet", True),
+    (255, 193, 4, 7, "pinned", True),      # odd cap: a last round of one iteration
+    (255, 193, 4, 2, "pinned", True),
+    (449, 389, 4, 6000, "pinned", True),
+    (1024, 1024, 4, 200, "pinned", True),  # one workgroup per CU
+])
+def test_mixed_shapes_bitwise(nx, ny, rows, maxiter, op, jacobi):
+    b = _rhs("normal", ny, nx)
+    print(f"[resident] mixed {nx}x{ny} rows={rows} cap={maxiter} {op} jacobi={jacobi}", flush=True)
+    ref = _solve(nx, ny, 1.0, 1.25, op, b, maxiter, "mixed", False, rows=rows, jacobi=jacobi, tol=1e-9)
+    new = _solve(nx, ny, 1.0, 1.25, op, b, maxiter, "mixed", True, rows=rows, jacobi=jacobi, tol=1e-9)
+    _same(new, ref)
+
+
+@pytest.mark.parametrize("kind", ["source", "tiny", "wide", "inf"])
+def test_mixed_values_bitwise(kind):
+    b = _rhs(kind, 97, 130)
+    if kind == "wide":
+        b = np.clip(b, -1e30, 1e30)
+    print(f"[resident] mixed values {kind}", flush=True)
+    ref = _solve(130, 97, 1.0, 1.0, "pinned", b, 200, "mixed", False)
+    new = _solve(130, 97, 1.0, 1.0, "pinned", b, 200, "mixed", True)
+    _same(new, ref)
+
+
+@pytest.mark.parametrize("nx,ny,precision", [(100, 70, "fp64"), (64, 64, "fp64"), (100, 70, "mixed"), (300, 200, "mixed")])
+def test_steps_bitwise(nx, ny, precision):
     """Steps of a lid-driven cavity, several per run and one per run."""
     from pyflow._device import cavity_params
     out = []
@@ -119,7 +155,7 @@ def test_fp64_steps_bitwise(nx, ny):
         p = cavity_params(nx, ny, dx=1.0, dy=1.0, scheme="quick", lid_velocity=1.0, Re=400.0, lin_tol=1e-8,
                           lin_maxiter=2000)
         print(f"[resident] steps {nx}x{ny} resident={resident}", flush=True)
-        b = _batch(p, "fp64", resident)
+        b = _batch(p, precision, resident)
         try:
             ds = [b.run(n)[0] for n in (3, 1, 2)]
             f = [np.zeros((ny + 2, nx + 2)) for _ in range(3)]
@@ -131,14 +167,15 @@ def test_fp64_steps_bitwise(nx, ny):
     assert out[0][1] == out[1][1]
 
 
-def test_fp64_meeting_fails_bitwise(monkeypatch):
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_meeting_fails_bitwise(monkeypatch, precision):
     """Workgroups that do not wait for each other (PYFLOW_MEET_US=0) run
     ordinary rounds wherever they did not all arrive at once: the same bits."""
     b = _rhs("normal", 260, 330)
-    ref = _solve(330, 260, 1.0, 1.0, "pinned", b, 300, "fp64", False)
+    ref = _solve(330, 260, 1.0, 1.0, "pinned", b, 300, precision, False)
     monkeypatch.setenv("PYFLOW_MEET_US", "0")
-    new = _solve(330, 260, 1.0, 1.0, "pinned", b, 300, "fp64", True)
-    print(f"[resident] no waiting: {new[2]} launches, one phase per launch {ref[2]}", flush=True)
+    new = _solve(330, 260, 1.0, 1.0, "pinned", b, 300, precision, True)
+    print(f"[resident] no waiting {precision}: {new[2]} launches, one phase per launch {ref[2]}", flush=True)
     _same(new, ref)
 
 
