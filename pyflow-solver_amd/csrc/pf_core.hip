@@ -481,6 +481,10 @@ static const void* round_fn_u(const pf_batch* b) {
   return b->multi ? round_fn_m<T, U, true>(b) : round_fn_m<T, U, false>(b);
 }
 
+static const void* res32_fn(int tpb) {
+  return tpb == 1 ? (const void*)k_round_res32<1> : tpb == 2 ? (const void*)k_round_res32<2> : (const void*)k_round_res32<4>;
+}
+
 static RoundLaunch round_launch(const pf_batch* b) {
   RoundLaunch L;
   L.blk = dim3(TX, TY);
@@ -491,7 +495,7 @@ static RoundLaunch round_launch(const pf_batch* b) {
       L.fn = b->multi ? (one ? (const void*)k_round_ca3<true, true> : (const void*)k_round_ca3<false, true>)
                       : (one ? (const void*)k_round_ca3<true, false> : (const void*)k_round_ca3<false, false>);
     } else if (b->res_kind == 2 && b->res_on)
-      L.fn = (const void*)k_round_res32;
+      L.fn = res32_fn(b->hcav[b->single_slot].tpb);
     else if (b->occ2)
       L.fn = b->single_slot >= 0 ? (const void*)k_round_occ2<true> : (const void*)k_round_occ2<false>;
     else
@@ -820,8 +824,8 @@ static int graph_len_of(int rounds) { return rounds <= 0 ? 0 : std::min(1024, st
 
 static int allow_region_lds() {
   const int bytes = std::max({region_lds_floats(8), ca_lds_floats(4), ca3_lds_floats(4), res32_lds_floats(4)}) * (int)sizeof(float);
-  const void* fns[17] = {
-      (const void*)k_round_res32,
+  const void* fns[19] = {
+      (const void*)k_round_res32<1>, (const void*)k_round_res32<2>, (const void*)k_round_res32<4>,
       (const void*)k_round_ca3<true, false>, (const void*)k_round_ca3<false, false>,
       (const void*)k_round_ca3<true, true>, (const void*)k_round_ca3<false, true>,
       (const void*)k_round_occ2<true>, (const void*)k_round_occ2<false>,

@@ -46,9 +46,10 @@ constexpr unsigned kMeetAbort = 0x10000u;
 
 // Layout of KArgs::res (bytes; every block starts on a 128-byte line).
 constexpr size_t kResMeet = 0;             // arrival words, one per round parity, 128 bytes apart
-constexpr size_t kResBcast = 512;          // kCopies lines of 16 words
-constexpr size_t kResPart = 4096;          // FP64: 2 x 3 x kResMaxBlk words; MIXED: 2 x kResMaxBlk lines of 16 words
-constexpr size_t kResFlag = kResPart + 2 * kResMaxBlk * 128;  // MIXED: a sequence number per workgroup, 128 bytes apart
+constexpr size_t kResBcast = 512;          // FP64: kCopies lines of 16 words
+constexpr size_t kResTotal = 2048;         // MIXED: kCopies lines of 2 KCA words (256 bytes each)
+constexpr size_t kResPart = 4096;          // FP64: 2 x 3 x kResMaxBlk words; MIXED: 4 x KCA x kResMaxBlk words
+constexpr size_t kResFlag = kResPart + 4 * KCA * kResMaxBlk * 8;  // MIXED: a sequence number per workgroup, 128 bytes apart
 constexpr size_t kResData = kResFlag + kResMaxBlk * 128;      // FP64: inboxes [2][nblk][4 sides][64]; MIXED: (r, p) [2][ny][nx]
 __host__ __device__ constexpr size_t res64_bytes(int nblk) { return kResData + (size_t)2 * nblk * 4 * 64 * 8; }
 __host__ __device__ constexpr size_t res32_bytes(size_t cells) { return kResData + 2 * cells * 8; }
@@ -74,9 +75,11 @@ __device__ inline void drain_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "mem
 struct ResShared {
   double val[2];          // FP64: alpha, beta
   float coef[4];          // MIXED: alpha_k, beta_k, alpha_k+1, beta_k+1
+  double tot[KCA];        // MIXED: totals of the round
+  double wtot[KCA][NWAVE];  // MIXED: wave totals
   double wsum[3][NWAVE];  // wave totals: P, and the two of Q
   unsigned seq0;        // sequence number of the last broadcast before this launch
-  int go, dead;
+  int go, dead, inc;
   int tiny[2];  // some d of the region or its ring is a tiny number, by iteration parity
 };
 
@@ -92,9 +95,11 @@ __device__ inline bool resident_enter(const KArgs& KA, const PfCav& C, int b, Re
     sh->tiny[0] = sh->tiny[1] = 0;
     if (nblk > 1) {
       unsigned* meet = (unsigned*)(KA.res + kResMeet + 128 * KA.parity);
-      const unsigned long long* line =
-          (const unsigned long long*)(KA.res + kResBcast) + 16 * (b & (kCopies - 1));
-      sh->seq0 = (unsigned)(dev_load(line) >> 32);
+      // The last sequence number: FP64 counts broadcasts, MIXED rounds (its flag).
+      const unsigned long long* last = (const unsigned long long*)(
+          C.prec == PF_PREC_MIXED ? KA.res + kResFlag + 128 * b : KA.res + kResBcast + 128 * (b & (kCopies - 1)));
+      const unsigned long long w = dev_load(last);
+      sh->seq0 = C.prec == PF_PREC_MIXED ? (unsigned)w : (unsigned)(w >> 32);
       drain_vmem();  // read before arriving: workgroup 0 broadcasts only after every arrival
       const long long t0 = wall_clock64();
       unsigned cur = __hip_atomic_fetch_add(meet, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
@@ -139,9 +144,9 @@ __device__ inline bool bcast_wait(const unsigned long long* line, int lane, int 
     if (wall_clock64() - t0 > kWaitTicks) return false;
   }
 }
-// The value of kSent-marked words q = lane + 64 t (t < 4, q < n), polled by one
-// whole wave; consumed words get kSent back. False after kWaitTicks.
-__device__ inline bool words_take(unsigned long long* w, int lane, int n, double (&v)[4]) {
+// The values of kSent-marked words q = lane + 64 t (t < 4, q < n), polled by one
+// whole wave. False after kWaitTicks.
+__device__ inline bool words_poll(const unsigned long long* w, int lane, int n, double (&v)[4]) {
   const long long t0 = wall_clock64();
   unsigned long long x[4];
   while (true) {
@@ -157,12 +162,15 @@ __device__ inline bool words_take(unsigned long long* w, int lane, int n, double
     if (wall_clock64() - t0 > kWaitTicks) return false;
   }
 #pragma unroll
+  for (int t = 0; t < 4; ++t) v[t] = __longlong_as_double((long long)x[t]);
+  return true;
+}
+__device__ inline void words_reset(unsigned long long* w, int lane, int n) {
+#pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int q = lane + 64 * t;
     if (q < n) dev_store(w + q, kSent);
-    v[t] = __longlong_as_double((long long)x[t]);
   }
-  return true;
 }
 // The fold of a round's preamble: per lane in increasing workgroup order, then
 // the DPP tree; the total is broadcast from lane 63.
@@ -388,7 +396,8 @@ __device__ __attribute__((always_inline)) inline void resident_cg64(const KArgs&
         bool ok = true;
         if (b == 0) {
           double v[4];
-          ok = words_take(pb, li, nblk, v);
+          ok = words_poll(pb, li, nblk, v);
+          words_reset(pb, li, nblk);
           pq = fold_words(li, nblk, v);
           alpha = rho / pq;
           const long long u = __double_as_longlong(alpha);
@@ -461,8 +470,10 @@ __device__ __attribute__((always_inline)) inline void resident_cg64(const KArgs&
         bool ok = true;
         if (b == 0) {
           double v[4], w[4];
-          ok = words_take(pb + kResMaxBlk, li, nblk, v);
-          ok = words_take(pb + 2 * kResMaxBlk, li, nblk, w) && ok;
+          ok = words_poll(pb + kResMaxBlk, li, nblk, v);
+          ok = words_poll(pb + 2 * kResMaxBlk, li, nblk, w) && ok;
+          words_reset(pb + kResMaxBlk, li, nblk);
+          words_reset(pb + 2 * kResMaxBlk, li, nblk);
           rho_prev = rho;
           rho = fold_words(li, nblk, v);
           rnorm2 = fold_words(li, nblk, w);
@@ -537,12 +548,10 @@ __device__ __attribute__((always_inline)) inline void resident_cg64(const KArgs&
   }
 }
 
-constexpr int kGatherPitch = kResMaxBlk + 1;
-// LDS of resident_ca: p, z = M r and M A p on a region with its 4-cell frame,
-// and the sums that workgroup 0 collects.
-__host__ __device__ constexpr int res32_lds_floats(int m) {
-  return (3 * (TY * m + 8) * HQ + 1) / 2 * 2 + 2 * KCA * kGatherPitch;
-}
+// LDS of resident_ca: p, z = M r and M A p on a region with its 4-cell frame.
+__host__ __device__ constexpr int res32_lds_floats(int m) { return 3 * (TY * m + 8) * HQ; }
+// Up to this many workgroups, each collects all sums itself.
+constexpr int kAllToAll = 16;
 
 // The two-iteration PCG rounds of an inner solve of a MIXED cavity (region_ca
 // and tail_ca, FP32 iterate), from a round that runs iterations to the round
@@ -560,16 +569,15 @@ __host__ __device__ constexpr int res32_lds_floats(int m) {
 // as the cell itself (its difference is +0, as region_ca's ghost copies make it).
 template <int M>
 __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& KA, const PfCav& C, PfScal& st,
-                                                                  double (*sm)[NPS], double* tot, ResShared& sh,
-                                                                  float* __restrict__ lds, int b) {
+                                                                  ResShared& sh, float* __restrict__ lds, int b) {
   constexpr int RH = TY * M, NR = RH + 8, TP = TY * HQ;
   constexpr int F1 = ca_frame_cells(RH, 1), F2 = ca_frame_cells(RH, 2), F3 = ca_frame_cells(RH, 3);
   constexpr int F4 = ca_frame_cells(RH, 4);
   static_assert(F3 <= NTH && F4 <= NTH + 64, "a frame cell per thread, and one more in wave 0");
+  static_assert(NR * HQ < (1 << 16), "LDS words fit 16 bits");
   float* __restrict__ lP = lds;
   float* __restrict__ lZ = lds + NR * HQ;
   float* __restrict__ lMA = lds + 2 * NR * HQ;
-  double* __restrict__ lG = (double*)(lds + (3 * NR * HQ + 1) / 2 * 2);  // [KCA][kGatherPitch]
   const int nx = C.nx, ny = C.ny, nblk = C.nblk, tiles_x = C.tiles_x;
   const int li = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
@@ -577,9 +585,9 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
   const int rx = b % tiles_x, ry = b / tiles_x;
   const int i0 = rx * TX, j0 = ry * RH;
   const int i = i0 + li;
-  const bool full = (i0 + TX <= nx) && (j0 + RH <= ny);
   const bool pinned = (C.op == 0);
   const float scx = pinned ? -C.cxf : C.cxf, scy = pinned ? -C.cyf : C.cyf;
+  const int rows = min(RH, ny - j0);  // rows of the region inside the domain
   auto minv = [&](int j, int ii) -> float {
     if (!C.jacobi) return 1.0f;
     return (ii == 0 || ii == nx - 1 || j == 0 || j == ny - 1) ? 1.0f : C.invdf;
@@ -587,201 +595,223 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
   auto ident = [&](int j, int ii) -> bool {
     return pinned ? (j == 0 && ii == 0) : (j == 0 || j == ny - 1 || ii == 0 || ii == nx - 1);
   };
-  auto lap = [&](const float* L, int o, int oe, int ow, int on, int os) -> float {
-    const float c = L[o];
+  auto lap = [&](const float* L, float c, int oe, int ow, int on, int os) -> float {
     return __fmul_rn((L[oe] - c) - (c - L[ow]), scx) + __fmul_rn((L[on] - c) - (c - L[os]), scy);
   };
-  const size_t n2 = (size_t)nx * ny;
-  const float* __restrict__ R = mixed_r(C, KA.parity);
-  const float* __restrict__ Pold = mixed_p(C, KA.parity ^ 1);
-  float* __restrict__ X = (float*)C.x;
-  unsigned long long* const xch = (unsigned long long*)(KA.res + kResData);
+  const unsigned n2 = (unsigned)(nx * ny);  // at most kResMaxBlk regions: below 2^21 cells
+  char* const xch = KA.res + kResData;
 
-  // Own cells.
+  // Own cells. East and west neighbours by offset (the cell itself where there
+  // is none); across the domain's lower and upper edge the wave that holds the
+  // edge row keeps a copy of it in the LDS row beyond (egS, egN: bit m).
   const int o0 = (wave + 4) * HQ + li + 4;
   const int oE = o0 + ((i + 1 < nx) ? 1 : 0), oW = o0 - ((i > 0) ? 1 : 0);
-  int oN[M], oS[M];
   float ro[M], po[M], xo[M], ao[M], cv[M], ev[M], mo[M];
-  unsigned inm = 0, idm = 0, pub = 0;  // in the domain; identity row; to be published (bit m)
-  const bool pubcol = (li < 4 && rx > 0) || (li >= TX - 4 && i0 + TX < nx);
+  unsigned idm = 0;              // identity rows (bit m)
+  unsigned inr = 0, egN = 0;     // wave-uniform: row m is in the domain; is its last row
+  const unsigned egS = (wave == 0 && j0 == 0) ? 1u : 0u;
+  {
+    const float* __restrict__ R = mixed_r(C, KA.parity);
+    const float* __restrict__ Pold = mixed_p(C, KA.parity ^ 1);
+    const float* __restrict__ X = (const float*)C.x;
 #pragma unroll
-  for (int m = 0; m < M; ++m) {
-    const int row = TY * m + wave, j = j0 + row;
-    const bool in = (i < nx) && (j < ny);
-    const size_t k = in ? (size_t)j * nx + i : 0;
-    ro[m] = R[k];
-    po[m] = Pold[k];
-    xo[m] = X[k];
-    mo[m] = minv(j, i);
-    oN[m] = o0 + m * TP + ((j + 1 < ny) ? HQ : 0);
-    oS[m] = o0 + m * TP - ((j > 0) ? HQ : 0);
-    if (in) {
-      inm |= 1u << m;
-      if (ident(j, i)) idm |= 1u << m;
-      if (pubcol || (row < 4 && j0 > 0) || (row >= RH - 4 && j0 + RH < ny)) pub |= 1u << m;
+    for (int m = 0; m < M; ++m) {
+      const int row = TY * m + wave, j = j0 + row;
+      const bool in = (i < nx) && (j < ny);
+      const unsigned k = in ? (unsigned)(j * nx + i) : 0u;
+      ro[m] = R[k];
+      po[m] = Pold[k];
+      xo[m] = X[k];
+      mo[m] = minv(j, i);
+      if (j < ny) inr |= 1u << m;
+      if (j == ny - 1) egN |= 1u << m;
+      if (in && ident(j, i)) idm |= 1u << m;
     }
   }
+  const bool full = (i0 + TX <= nx) && rows == RH;
+  const bool edges = (egS | egN) != 0;
   const bool any_id = __any(idm != 0);
+  auto own_put = [&](float* L, int m, float v) {
+    if ((inr >> m) & 1u) L[o0 + m * TP] = v;
+    if (edges) {
+      if ((egN >> m) & 1u) L[o0 + m * TP + HQ] = v;
+      if ((egS >> m) & 1u) L[o0 + m * TP - HQ] = v;
+    }
+  };
   // Frame cells: q0 per thread, counted down so that wave 0, which also waits
-  // for the broadcasts, has the outermost; q1 in wave 0 where the frame has more
-  // than NTH cells.
+  // for the totals, has the outermost; q1 in wave 0 where the frame has more
+  // than NTH cells. f: LDS word; bits 16-19 the neighbours it has (E, W, N, S),
+  // 20 identity row, 21-23 within distance 1, 2, 3, 24 received (3 or 4).
   const int q0 = NTH - 1 - tid;
-  int fo = 0, fE = 0, fW = 0, fN = 0, fS = 0;
-  bool fin = false, fid = false;
+  unsigned f = 0, fk = 0, g = 0, gk = 0;  // fk, gk: byte offsets in the exchange buffers
   float fr = 0.f, fp = 0.f, fa = 0.f, fc = 0.f, fe = 0.f, fm = 0.f;
-  size_t fk = 0;
-  if (q0 < F4) {
-    int row, col;
-    ca_frame_cell(RH, q0, row, col);
-    const int gj = j0 + row - 4, gi = i0 + col - 4;
-    fin = gi >= 0 && gi < nx && gj >= 0 && gj < ny;
-    if (fin) {
-      fo = row * HQ + col;
-      fE = fo + ((gi + 1 < nx) ? 1 : 0);
-      fW = fo - ((gi > 0) ? 1 : 0);
-      fN = fo + ((gj + 1 < ny) ? HQ : 0);
-      fS = fo - ((gj > 0) ? HQ : 0);
-      fid = ident(gj, gi);
+  {
+    const float* __restrict__ R = mixed_r(C, KA.parity);
+    const float* __restrict__ Pold = mixed_p(C, KA.parity ^ 1);
+    int row = 0, col = 0;
+    if (q0 < F4) ca_frame_cell(RH, q0, row, col);
+    int gj = j0 + row - 4, gi = i0 + col - 4;
+    if (q0 < F4 && gi >= 0 && gi < nx && gj >= 0 && gj < ny) {
+      f = (unsigned)(row * HQ + col);
+      if (gi + 1 < nx) f |= 1u << 16;
+      if (gi > 0) f |= 1u << 17;
+      if (gj + 1 < ny) f |= 1u << 18;
+      if (gj > 0) f |= 1u << 19;
+      if (ident(gj, gi)) f |= 1u << 20;
+      if (q0 < F1) f |= 1u << 21;
+      if (q0 < F2) f |= 1u << 22;
+      if (q0 < F3) f |= 1u << 23;
+      if (q0 >= F2) f |= 1u << 24;
       fm = minv(gj, gi);
-      fk = (size_t)gj * nx + gi;
-      fr = R[fk];
-      fp = Pold[fk];
+      const unsigned k = (unsigned)(gj * nx + gi);
+      fk = 8 * k;
+      fr = R[k];
+      fp = Pold[k];
+      lP[f & 0xffffu] = fp;
+      lZ[f & 0xffffu] = fm * fr;
+    }
+    if (F4 > NTH && NTH + tid < F4) {
+      ca_frame_cell(RH, NTH + tid, row, col);
+      gj = j0 + row - 4;
+      gi = i0 + col - 4;
+      if (gi >= 0 && gi < nx && gj >= 0 && gj < ny) {
+        g = (unsigned)(row * HQ + col) | (1u << 24);
+        const unsigned k = (unsigned)(gj * nx + gi);
+        gk = 8 * k;
+        lP[g & 0xffffu] = Pold[k];
+        lZ[g & 0xffffu] = minv(gj, gi) * R[k];
+      }
     }
   }
-  const bool fin1 = fin && q0 < F1, fin2 = fin && q0 < F2, fin3 = fin && q0 < F3, finX = fin && q0 >= F2;
-  int go1 = 0;  // q1: LDS word and grid cell
-  bool gin = false;
-  float gm = 0.f, gr = 0.f, gp = 0.f;
-  size_t gk = 0;
-  if (F4 > NTH && NTH + tid < F4) {
-    int row, col;
-    ca_frame_cell(RH, NTH + tid, row, col);
-    const int gj = j0 + row - 4, gi = i0 + col - 4;
-    gin = gi >= 0 && gi < nx && gj >= 0 && gj < ny;
-    if (gin) {
-      go1 = row * HQ + col;
-      gm = minv(gj, gi);
-      gk = (size_t)gj * nx + gi;
-      gr = R[gk];
-      gp = Pold[gk];
+  // The cell this thread publishes after every round, if any (e: LDS word, bit
+  // 24 set). A neighbour's frame at distances 3 and 4 needs the region's rows
+  // and columns 2 and 3 from each side that has a neighbour.
+  unsigned e = 0, ek = 0;
+  {
+    int row = -1, col = 0;
+    if (tid < 4 * TX) {
+      const int t = tid / TX;
+      row = t < 2 ? 2 + t : RH - 6 + t;
+      col = tid % TX;
+    } else if (tid < 4 * TX + 4 * (RH - 4)) {
+      const int q = tid - 4 * TX, t = q / (RH - 4), k = q % (RH - 4);
+      col = t < 2 ? 2 + t : TX - 6 + t;
+      row = k < 2 ? k : (k < RH - 6 ? k + 2 : k + 4);
+    }
+    const bool byrow = ((row == 2 || row == 3) && j0 > 0) || ((row == RH - 4 || row == RH - 3) && j0 + RH < ny);
+    const bool bycol = ((col == 2 || col == 3) && rx > 0) || ((col == TX - 4 || col == TX - 3) && i0 + TX < nx);
+    if (row >= 0 && (byrow || bycol) && row < rows && i0 + col < nx) {
+      e = (unsigned)((row + 4) * HQ + col + 4) | (1u << 24);
+      ek = 8 * (unsigned)((j0 + row) * nx + i0 + col);
     }
   }
-  const bool loads = __any(finX || gin);  // this wave receives frame cells
-  // The neighbour whose sequence number lane 0..7 watches.
-  const unsigned long long* flag = nullptr;
-  unsigned long long* const flags = (unsigned long long*)(KA.res + kResFlag);
+  // The neighbour whose sequence number lane 0..7 of wave 15 watches, else the
+  // region itself.
+  int watch = b;
   if (li < 8) {
     const int t = li < 4 ? li : li + 1;  // 3 x 3 without the centre
-    const int ex = t % 3 - 1, ey = t / 3 - 1;
-    const int nxr = rx + ex, nyr = ry + ey;
-    if (nxr >= 0 && nxr < tiles_x && nyr >= 0 && nyr * RH < ny) flag = flags + (size_t)(nyr * tiles_x + nxr) * 16;
+    const int nxr = rx + t % 3 - 1, nyr = ry + t / 3 - 1;
+    if (nxr >= 0 && nxr < tiles_x && nyr >= 0 && nyr * RH < ny) watch = nyr * tiles_x + nxr;
   }
-  unsigned long long* const part = (unsigned long long*)(KA.res + kResPart);
-  unsigned long long* const bcast = (unsigned long long*)(KA.res + kResBcast);
-  unsigned long long* const line = bcast + 16 * (b & (kCopies - 1));
   const unsigned seq0 = sh.seq0;
+  // Which slots this wave collects: every workgroup all of them (wave k slot k),
+  // or workgroup b the slots k = b mod nown, in waves 8 and up.
+  const bool multi = nblk > 1, all = nblk <= kAllToAll;
+  const int nown = min(nblk, KCA);
+  const int slot = all ? wave : (wave >= 8 && b < nown ? b + (wave - 8) * nown : KCA);
+  int it_total = st.it_total, inc = st.ca_inc;
 
   // The stencils of the first basis.
-  auto own_put = [&](float* L, const float (&v)[M]) {
 #pragma unroll
-    for (int m = 0; m < M; ++m) L[o0 + m * TP] = v[m];
-  };
-  {
-    float z[M];
-#pragma unroll
-    for (int m = 0; m < M; ++m) z[m] = mo[m] * ro[m];
-    own_put(lP, po);
-    own_put(lZ, z);
-  }
-  if (fin) {
-    lP[fo] = fp;
-    lZ[fo] = fm * fr;
-  }
-  if (gin) {
-    lP[go1] = gp;
-    lZ[go1] = gm * gr;
+  for (int m = 0; m < M; ++m) {
+    own_put(lP, m, po[m]);
+    own_put(lZ, m, mo[m] * ro[m]);
   }
   __syncthreads();
   auto own_a = [&]() {  // a = A p, M a into LDS
 #pragma unroll
-    for (int m = 0; m < M; ++m) ao[m] = lap(lP, o0 + m * TP, oE + m * TP, oW + m * TP, oN[m], oS[m]);
-    if (any_id) {
-#pragma unroll
-      for (int m = 0; m < M; ++m)
-        if ((idm >> m) & 1u) ao[m] = po[m];
+    for (int m = 0; m < M; ++m) {
+      const int d = m * TP;
+      ao[m] = lap(lP, po[m], oE + d, oW + d, o0 + d + HQ, o0 + d - HQ);
+      if (any_id) ao[m] = ((idm >> m) & 1u) ? po[m] : ao[m];
+      own_put(lMA, m, mo[m] * ao[m]);
     }
-#pragma unroll
-    for (int m = 0; m < M; ++m) lMA[o0 + m * TP] = mo[m] * ao[m];
   };
   auto own_ce = [&](int m) {  // c = A M a, e = A z
-    cv[m] = lap(lMA, o0 + m * TP, oE + m * TP, oW + m * TP, oN[m], oS[m]);
-    ev[m] = lap(lZ, o0 + m * TP, oE + m * TP, oW + m * TP, oN[m], oS[m]);
-    if (any_id && ((idm >> m) & 1u)) {
-      cv[m] = mo[m] * ao[m];
-      ev[m] = mo[m] * ro[m];
+    const int d = m * TP;
+    const float ma = mo[m] * ao[m], z = mo[m] * ro[m];
+    cv[m] = lap(lMA, ma, oE + d, oW + d, o0 + d + HQ, o0 + d - HQ);
+    ev[m] = lap(lZ, z, oE + d, oW + d, o0 + d + HQ, o0 + d - HQ);
+    if (any_id) {
+      cv[m] = ((idm >> m) & 1u) ? ma : cv[m];
+      ev[m] = ((idm >> m) & 1u) ? z : ev[m];
     }
   };
+  auto frame_lap = [&](const float* L, float c) -> float {
+    const int o = f & 0xffffu;
+    const float v = lap(L, c, o + ((f >> 16) & 1u), o - ((f >> 17) & 1u), o + ((f >> 18) & 1u) * HQ,
+                        o - ((f >> 19) & 1u) * HQ);
+    return (f & (1u << 20)) ? c : v;
+  };
   auto frame_a = [&]() {
-    const float v = lap(lP, fo, fE, fW, fN, fS);
-    fa = fid ? fp : v;
-    lMA[fo] = fm * fa;
+    fa = frame_lap(lP, fp);
+    lMA[f & 0xffffu] = fm * fa;
   };
   auto frame_ce = [&]() {
-    const float v = lap(lMA, fo, fE, fW, fN, fS), w = lap(lZ, fo, fE, fW, fN, fS);
-    fc = fid ? fm * fa : v;
-    fe = fid ? fm * fr : w;
+    fc = frame_lap(lMA, fm * fa);
+    fe = frame_lap(lZ, fm * fr);
   };
   own_a();
-  if (fin3) frame_a();
+  if (f & (1u << 23)) frame_a();
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < M; ++m) own_ce(m);
-  if (fin2) frame_ce();
+  if (f & (1u << 22)) frame_ce();
   float a0 = (float)st.ca0, b0 = (float)st.cb0, a1 = (float)st.ca1, b1 = (float)st.cb1;
   __syncthreads();
   bool dead = false;
   int n = 0;
   while (true) {
     const unsigned seq = seq0 + 1 + (unsigned)n;
+    char* const xb = xch + ((n & 1) ? (size_t)n2 * 8 : 0);
     // The two steps (ca_steps).
-    unsigned long long* const xb = xch + (n & 1) * n2;
 #pragma unroll
     for (int m = 0; m < M; ++m) {
       const float z = mo[m] * ro[m], ma = mo[m] * ao[m];
       const float p1 = (z - a0 * ma) + b0 * po[m];
       const float ap1 = (ev[m] - a0 * cv[m]) + b0 * ao[m];
-      const float r2 = (ro[m] - a0 * ao[m]) - a1 * ap1;
-      const float z2 = mo[m] * r2;
-      const float p2 = z2 + b1 * p1;
       xo[m] = (xo[m] + a0 * po[m]) + a1 * p1;
-      ro[m] = r2;
-      po[m] = p2;
-      lP[o0 + m * TP] = p2;
-      lZ[o0 + m * TP] = z2;
-      if ((pub >> m) & 1u)
-        dev_store(xb + (size_t)(j0 + TY * m + wave) * nx + i,
-                  (unsigned long long)__float_as_uint(r2) | ((unsigned long long)__float_as_uint(p2) << 32));
+      ro[m] = (ro[m] - a0 * ao[m]) - a1 * ap1;
+      const float z2 = mo[m] * ro[m];
+      po[m] = z2 + b1 * p1;
+      own_put(lP, m, po[m]);
+      own_put(lZ, m, z2);
     }
-    if (fin2) {
+    if (f & (1u << 22)) {
       const float z = fm * fr, ma = fm * fa;
       const float p1 = (z - a0 * ma) + b0 * fp;
       const float ap1 = (fe - a0 * fc) + b0 * fa;
       fr = (fr - a0 * fa) - a1 * ap1;
       const float z2 = fm * fr;
       fp = z2 + b1 * p1;
-      lP[fo] = fp;
-      lZ[fo] = z2;
+      lP[f & 0xffffu] = fp;
+      lZ[f & 0xffffu] = z2;
     }
     __syncthreads();
+    if (e) {
+      const unsigned o = e & 0xffffu;
+      dev_store((unsigned long long*)(xb + ek),
+                (unsigned long long)__float_as_uint(lZ[o]) | ((unsigned long long)__float_as_uint(lP[o]) << 32));
+    }
     own_a();
-    if (fin1) frame_a();
+    if (f & (1u << 21)) frame_a();
     __syncthreads();
     // c, e and the Gram sums of the new basis (pass 5 of region_ca).
     double acc[NP] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int m = 0; m < M; ++m) {
       own_ce(m);
-      if (full || ((inm >> m) & 1u)) {
+      if (full || (((inr >> m) & 1u) && i < nx)) {
         const double p2 = po[m], z2 = mo[m] * ro[m], r2 = ro[m], a2 = ao[m];
         const double ma2 = mo[m] * ao[m], c2 = cv[m], mc2 = mo[m] * cv[m], e2 = ev[m], me2 = mo[m] * ev[m];
         acc[0] = __fma_rn(p2, a2, acc[0]);
@@ -800,112 +830,105 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
         acc[13] = __fma_rn(r2, r2, acc[13]);
       }
     }
-    wave_partials_ca(acc, sm);
+    wave_partials_ca(acc, [&](int k, double v) { sh.wtot[k][wave] = v; });
     drain_vmem();  // the published cells are in memory before the barrier, so before the flag
     __syncthreads();
-    unsigned long long* const pb = part + (size_t)(n & 1) * kResMaxBlk * 16;
+    unsigned long long* const pb = (unsigned long long*)(KA.res + kResPart) + (size_t)(seq & 3) * KCA * kResMaxBlk;
     if (tid < KCA) {
-      double t = sm[0][tid];
-#pragma unroll
-      for (int w = 1; w < NWAVE; ++w) t += sm[w][tid];
-      dev_store_f64(pb + 16 * b + tid, t);
+      const double t = fold_waves(sh.wtot[tid]);
+      if (multi)
+        dev_store_f64(pb + tid * kResMaxBlk + b, t);
+      else
+        sh.tot[tid] = 0.0 + t;
     }
-    if (tid == NTH - 1) dev_store(flags + 16 * b, (unsigned long long)seq);
-    // The frame at distances 3 and 4.
-    if (loads) {
-      const long long t0 = wall_clock64();
-      while (true) {
-        const unsigned f = flag ? (unsigned)dev_load(flag) : seq;
-        if (!__any((int)(f - seq) < 0)) break;
-        if (wall_clock64() - t0 > kWaitTicks) {
-          if (li == 0) sh.dead = 1;
-          break;
+    if (multi) {
+      if (wave == NWAVE - 1) {
+        unsigned long long* const flags = (unsigned long long*)(KA.res + kResFlag);
+        if (li == 0) dev_store(flags + 16 * b, (unsigned long long)seq);
+        const long long t0 = wall_clock64();
+        while (true) {
+          const unsigned w = li < 8 ? (unsigned)dev_load(flags + 16 * watch) : seq;
+          if (!__any((int)(w - seq) < 0)) break;
+          if (wall_clock64() - t0 > kWaitTicks) {
+            if (li == 0) sh.dead = 1;
+            break;
+          }
         }
       }
-      asm volatile("" ::: "memory");  // the frame is loaded after its flags were seen
-    }
-    unsigned long long fx = 0, gx = 0;
-    if (finX) fx = dev_load(xb + fk);
-    if (gin) gx = dev_load(xb + gk);
-    if (b == 0) {  // collect the sums
-      unsigned long long x[4];
-      const long long t0 = wall_clock64();
-      while (true) {
-        bool miss = false;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int w = tid + NTH * t;
-          x[t] = ((w >> 4) < nblk && (w & 15) < KCA) ? dev_load(pb + w) : 0ull;
+      __syncthreads();  // the neighbours' cells are in memory
+      unsigned long long fx = 0, gx = 0;
+      if (f & (1u << 24)) fx = dev_load((const unsigned long long*)(xb + fk));
+      if (g) gx = dev_load((const unsigned long long*)(xb + gk));
+      if (slot < KCA) {
+        bool ok = true;
+        for (int k = slot; k < KCA; k += all ? KCA : 8 * nown) {
+          double v[4];
+          ok = words_poll(pb + k * kResMaxBlk, li, nblk, v) && ok;
+          const double t = fold_words(li, nblk, v);
+          if (all) {
+            if (li == 0) sh.tot[k] = t;
+          } else {
+            const unsigned long long u = (unsigned long long)__double_as_longlong(t);
+            const unsigned pay = (li & 1) ? (unsigned)(u >> 32) : (unsigned)u;
+            unsigned long long* const total = (unsigned long long*)(KA.res + kResTotal);
+            if (li < 2 * kCopies) dev_store(total + 32 * (li >> 1) + 2 * k + (li & 1), pay | ((unsigned long long)seq << 32));
+            words_reset(pb + k * kResMaxBlk, li, nblk);
+          }
         }
-#pragma unroll
-        for (int t = 0; t < 4; ++t) miss |= x[t] == kSent;
-        if (!__any(miss)) break;
-        if (wall_clock64() - t0 > kWaitTicks) {
-          if (li == 0) sh.dead = 1;
-          break;
-        }
+        if (!ok && li == 0) sh.dead = 1;
       }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int w = tid + NTH * t;
-        if ((w >> 4) < nblk && (w & 15) < KCA) {
-          lG[(w & 15) * kGatherPitch + (w >> 4)] = __longlong_as_double((long long)x[t]);
-          dev_store(pb + w, kSent);
-        }
+      // Each workgroup puts its own words of the round before (the last one of
+      // the launch before, if this is the first) back to kSent: every workgroup has
+      // read them, since all have stored this round's.
+      if (all && tid < KCA)
+        dev_store((unsigned long long*)(KA.res + kResPart) + ((size_t)((seq + 3) & 3) * KCA + tid) * kResMaxBlk + b, kSent);
+      if (f & (1u << 24)) {
+        fp = __uint_as_float((unsigned)(fx >> 32));
+        lZ[f & 0xffffu] = __uint_as_float((unsigned)fx);
+        lP[f & 0xffffu] = fp;
       }
-    }
-    if (finX) {
-      fr = __uint_as_float((unsigned)fx);
-      fp = __uint_as_float((unsigned)(fx >> 32));
-      lP[fo] = fp;
-      lZ[fo] = fm * fr;
-    }
-    if (gin) {
-      lP[go1] = __uint_as_float((unsigned)(gx >> 32));
-      lZ[go1] = gm * __uint_as_float((unsigned)gx);
+      if (g) {
+        lP[g & 0xffffu] = __uint_as_float((unsigned)(gx >> 32));
+        lZ[g & 0xffffu] = __uint_as_float((unsigned)gx);
+      }
     }
     __syncthreads();
-    if (b == 0 && wave < KCA) {
-      double v = 0.0;
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-        if (li + 64 * t < nblk) v = v + lG[wave * kGatherPitch + li + 64 * t];
-      v = wave_reduce<false>(v);
-      if (li == 63) tot[wave] = v;
-    }
-    if (fin3 && !fin1) frame_a();
+    if ((f & (5u << 21)) == (4u << 21)) frame_a();  // distances 2 and 3
     __syncthreads();
+    it_total += inc;
     if (wave == 0) {
-      bool ok = true;
-      if (b == 0) {
-        if (li == 63) {
-          tail_ca(C, st, tot);
-          sh.go = (st.phase == PH_CG && n + 1 < kResIters) ? 1 : 0;
-          sh.coef[0] = (float)st.ca0;
-          sh.coef[1] = (float)st.cb0;
-          sh.coef[2] = (float)st.ca1;
-          sh.coef[3] = (float)st.cb1;
-        }
-        const int wd = li & 7;
-        drain_vmem();  // the collected words are back at kSent
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // lane 63's results, within the wave
-        const unsigned pay = wd < 4 ? __float_as_uint(sh.coef[wd]) : (unsigned)sh.go;
-        if (wd < 5) dev_store(bcast + 16 * (li >> 3) + wd, pay | ((unsigned long long)seq << 32));
-      } else {
+      if (!all) {
         unsigned pay;
-        ok = bcast_wait(line, li, 5, seq, pay);
-        if (li < 4) sh.coef[li] = __uint_as_float(pay);
-        if (li == 4) sh.go = (int)pay;
+        const unsigned long long* const line = (const unsigned long long*)(KA.res + kResTotal) + 32 * (b & (kCopies - 1));
+        const bool ok = bcast_wait(line, li, 2 * KCA, seq, pay);
+        if (li < 2 * KCA) ((unsigned*)sh.tot)[li] = pay;
+        if (!ok && li == 0) sh.dead = 1;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       }
-      if (!ok && li == 0) sh.dead = 1;
+      const CaTail r = tail_ca_steps(sh.tot, it_total, C.maxiter, st.inner_atol);
+      if (li == 0) {
+        sh.coef[0] = (float)r.a0;
+        sh.coef[1] = (float)r.b0;
+        sh.coef[2] = (float)r.a1;
+        sh.coef[3] = (float)r.b1;
+        sh.inc = r.n;
+        sh.go = (r.next == 0 && n + 1 < kResIters) ? 1 : 0;
+        if (b == 0 && sh.go == 0) {
+          st.it += it_total - st.it_total;
+          st.it_run += it_total - st.it_total;
+          st.it_total = it_total;
+          tail_ca_store(C, st, sh.tot, r);
+        }
+      }
     }
-    if (fin2) frame_ce();
+    if (f & (1u << 22)) frame_ce();
     n += 1;
     __syncthreads();
     a0 = sh.coef[0];
     b0 = sh.coef[1];
     a1 = sh.coef[2];
     b1 = sh.coef[3];
+    inc = sh.inc;
     dead = sh.dead != 0;
     if (dead || sh.go == 0) break;
   }
@@ -916,10 +939,12 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
   // Leave the vectors as a round of this parity leaves them.
   float* __restrict__ Rn = mixed_r(C, KA.parity ^ 1);
   float* __restrict__ Pn = mixed_p(C, KA.parity);
+  float* __restrict__ X = (float*)C.x;
 #pragma unroll
   for (int m = 0; m < M; ++m) {
-    if ((inm >> m) & 1u) {
-      const size_t k = (size_t)(j0 + TY * m + wave) * nx + i;
+    const int j = j0 + TY * m + wave;
+    if (i < nx && j < ny) {
+      const unsigned k = (unsigned)(j * nx + i);
       Rn[k] = ro[m];
       Pn[k] = po[m];
       X[k] = xo[m];

@@ -370,23 +370,18 @@ __device__ __attribute__((always_inline)) inline void tail_cg_xd(const PfCav& C,
 //   z_k+2 = z_k+1 - alpha_k+1 T p_k+1,  beta_k+1 = z_k+2.W.z_k+2 / gamma_k+1
 // W is a weighted Gram matrix, symmetric whatever A is, so the identity rows
 // of the pinned and Dirichlet operators need no special case.
-__device__ __attribute__((always_inline)) inline void tail_ca(const PfCav& C, PfScal& S, const double* t) {
-  S.pending = PH_IDLE;
-  const int inc = S.ca_inc;
-  S.it += inc;
-  S.it_total += inc;
-  S.it_run += inc;
-  S.rnorm2 = t[13];
-  S.rho = t[10];
-  if (S.it_total >= C.maxiter) {
-    S.info = C.maxiter;
-    S.phase = outer_entry(C);
-    return;
-  }
-  if (sqrt(S.rnorm2) < S.inner_atol) {
-    S.phase = outer_entry(C);
-    return;
-  }
+struct CaTail {
+  double a0, b0, a1, b1;
+  int n;     // iterations of the next round
+  int next;  // 0: the next round iterates; 1: the iteration budget is spent; 2: the inner tolerance is met
+};
+__device__ __attribute__((always_inline)) inline CaTail tail_ca_steps(const double* t, int it_total, int maxiter,
+                                                                      double inner_atol) {
+  CaTail r;
+  r.a0 = r.b0 = r.a1 = r.b1 = 0.0;
+  r.n = 0;
+  r.next = it_total >= maxiter ? 1 : (sqrt(t[13]) < inner_atol ? 2 : 0);
+  if (r.next) return r;
   const double w01 = t[0], w02 = t[1], w04 = t[2], w11 = t[3], w12 = t[4], w13 = t[5], w14 = t[6];
   const double w22 = t[7], w23 = t[8], w24 = t[9], w33 = t[10], w34 = t[11], w44 = t[12];
   double a0 = w33 / w01;
@@ -404,7 +399,7 @@ __device__ __attribute__((always_inline)) inline void tail_ca(const PfCav& C, Pf
     const double pap = (w34 - a0 * w23 + b0 * w13) + (-a0 * w14 + a0 * a0 * w12 - a0 * b0 * w11) +
                        (b0 * w04 - a0 * b0 * w02 + b0 * b0 * w01);
     const double a1c = g1 / pap;
-    if (C.maxiter - S.it_total >= 2 && g1 > 0.0 && pap != 0.0 && isfinite(a1c)) {
+    if (maxiter - it_total >= 2 && g1 > 0.0 && pap != 0.0 && isfinite(a1c)) {
       a1 = a1c;
       n = 2;
       const double k1 = -(a0 + a1 * b0), k2 = a1 * a0, k4 = -a1;
@@ -415,14 +410,40 @@ __device__ __attribute__((always_inline)) inline void tail_ca(const PfCav& C, Pf
     }
     if (!isfinite(b0)) b0 = 0.0;
   }
-  S.ca0 = a0;
-  S.cb0 = b0;
-  S.ca1 = a1;
-  S.cb1 = b1;
-  S.ca_inc = n;
-  S.alpha = n == 2 ? a1 : a0;
-  S.beta = n == 2 ? b1 : b0;
+  r.a0 = a0;
+  r.b0 = b0;
+  r.a1 = a1;
+  r.b1 = b1;
+  r.n = n;
+  return r;
+}
+// The state after the tail of a round that left the totals t and ran S.ca_inc
+// iterations.
+__device__ __attribute__((always_inline)) inline void tail_ca_store(const PfCav& C, PfScal& S, const double* t,
+                                                                    const CaTail& r) {
+  S.pending = PH_IDLE;
+  S.rnorm2 = t[13];
+  S.rho = t[10];
+  if (r.next) {
+    if (r.next == 1) S.info = C.maxiter;
+    S.phase = outer_entry(C);
+    return;
+  }
+  S.ca0 = r.a0;
+  S.cb0 = r.b0;
+  S.ca1 = r.a1;
+  S.cb1 = r.b1;
+  S.ca_inc = r.n;
+  S.alpha = r.n == 2 ? r.a1 : r.a0;
+  S.beta = r.n == 2 ? r.b1 : r.b0;
   S.phase = PH_CG;
+}
+__device__ __attribute__((always_inline)) inline void tail_ca(const PfCav& C, PfScal& S, const double* t) {
+  const int inc = S.ca_inc;
+  S.it += inc;
+  S.it_total += inc;
+  S.it_run += inc;
+  tail_ca_store(C, S, t, tail_ca_steps(t, S.it_total, C.maxiter, S.inner_atol));
 }
 
 // Tail of a three-iteration round (s = 3). The pending round's basis is
@@ -2043,10 +2064,11 @@ __device__ __attribute__((always_inline)) inline double swap_sum(double x, doubl
   const double ys = __longlong_as_double((long long)((unsigned long long)lo[1] | ((unsigned long long)hi[1] << 32)));
   return xs + ys;
 }
-__device__ __attribute__((always_inline)) inline void wave_partials_ca(double (&v)[NP], double (*sm)[NPS]) {
+template <class F>
+__device__ __attribute__((always_inline)) inline void wave_partials_ca(double (&v)[NP], F put) {
   static_assert(KCA <= 16 && NP >= 16, "16 slots carried through the exchange");
   const int tid = tid_flat();
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63;
 #pragma unroll
   for (int k = KCA; k < 16; ++k) v[k] = 0.0;
   double a[8], b[4], c[2];
@@ -2077,11 +2099,11 @@ __device__ __attribute__((always_inline)) inline void wave_partials_ca(double (&
   d = d + dpp_full<0x4E>(d);  // quad_perm [2,3,0,1]
   d = d + dpp_full<0xB1>(d);  // quad_perm [1,0,3,2]
   const int q = lane >> 2;
-  if ((lane & 3) == 0 && q < KCA) sm[wave][q] = d;
+  if ((lane & 3) == 0 && q < KCA) put(q, d);
 }
 __device__ inline void block_partials_ca(double (&v)[NP], double (*sm)[NPS], double* dst, int stride) {
   const int tid = tid_flat();
-  wave_partials_ca(v, sm);
+  wave_partials_ca(v, [&](int q, double d) { sm[tid >> 6][q] = d; });
   __syncthreads();
   if (tid < KCA) {
     double t = sm[0][tid];
@@ -2628,7 +2650,7 @@ __device__ __attribute__((always_inline)) inline void round_body_ca(const KArgs&
   }
   if constexpr (RES) {
     if (phase == PH_CG && st.ca_inc > 0 && resident_enter(KA, C, b, rsh)) {
-      resident_ca<M>(KA, C, st, sm, tot, *rsh, lds, b);
+      resident_ca<M>(KA, C, st, *rsh, lds, b);
       if (b == 0) {
         __syncthreads();
         if (tid == 0 && !st.dsetup) st.rounds_run += 1;
@@ -2891,23 +2913,21 @@ __global__ __launch_bounds__(NTH) void k_round_res64(const KArgs KA) {
 }
 
 // The same for single MIXED cavities with an FP32 iterate and two PCG
-// iterations per round.
+// iterations per round, on regions of M tiles (a kernel each, so that none's
+// registers pay for another's code).
+template <int M>
 __global__ __launch_bounds__(NTH) void k_round_res32(const KArgs KA) {
   __shared__ PfScal st;
   __shared__ double sm[NWAVE][NPS];
   __shared__ double tot[NPS];
   __shared__ ResShared rsh;
-  extern __shared__ float lds_dyn[];  // ca_lds_floats(tpb) or res32_lds_floats(tpb) floats
+  extern __shared__ float lds_dyn[];  // ca_lds_floats(M) or res32_lds_floats(M) floats
   const PfCav& C = KA.cav0;
   const PfCav* Cg = KA.cavs + KA.slot0;
   const int lg = blockIdx.x - C.blk0;
   const int b = ((C.blk0 & 7) == 0 && (C.nblk & 7) == 0) ? (lg & 7) * (C.nblk >> 3) + (lg >> 3) : lg;
   if (b == 0 && tid_flat() == 0) resident_clear_meet(KA);
-  switch (C.tpb) {
-    case 1: round_body_ca<1, false, false, 3, true>(KA, C, Cg, KA.slot0, b, st, sm, tot, lds_dyn, &rsh); break;
-    case 2: round_body_ca<2, false, false, 3, true>(KA, C, Cg, KA.slot0, b, st, sm, tot, lds_dyn, &rsh); break;
-    default: round_body_ca<4, false, false, 3, true>(KA, C, Cg, KA.slot0, b, st, sm, tot, lds_dyn, &rsh); break;
-  }
+  round_body_ca<M, false, false, 3, true>(KA, C, Cg, KA.slot0, b, st, sm, tot, lds_dyn, &rsh);
 }
 
 // Batches whose cavities all run three PCG iterations per round (PfCav::ca
