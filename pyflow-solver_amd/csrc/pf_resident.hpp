@@ -548,8 +548,9 @@ __device__ __attribute__((always_inline)) inline void resident_cg64(const KArgs&
   }
 }
 
-// LDS of resident_ca: p, z = M r and M A p on a region with its 4-cell frame.
-__host__ __device__ constexpr int res32_lds_floats(int m) { return 3 * (TY * m + 8) * HQ; }
+// LDS of resident_ca: p, z = M r and M A p on a region with its 4-cell frame,
+// and x of its cells.
+__host__ __device__ constexpr int res32_lds_floats(int m) { return 3 * (TY * m + 8) * HQ + m * NTH; }
 // Up to this many workgroups, each collects all sums itself.
 constexpr int kAllToAll = 16;
 
@@ -578,6 +579,7 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
   float* __restrict__ lP = lds;
   float* __restrict__ lZ = lds + NR * HQ;
   float* __restrict__ lMA = lds + 2 * NR * HQ;
+  float* __restrict__ lX = lds + 3 * NR * HQ + threadIdx.y * TX + threadIdx.x;  // cell m at lX[m * NTH]
   const int nx = C.nx, ny = C.ny, nblk = C.nblk, tiles_x = C.tiles_x;
   const int li = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
@@ -606,7 +608,7 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
   // edge row keeps a copy of it in the LDS row beyond (egS, egN: bit m).
   const int o0 = (wave + 4) * HQ + li + 4;
   const int oE = o0 + ((i + 1 < nx) ? 1 : 0), oW = o0 - ((i > 0) ? 1 : 0);
-  float ro[M], po[M], xo[M], ao[M], cv[M], ev[M], mo[M];
+  float ro[M], po[M], ao[M], cv[M], ev[M], mo[M];
   unsigned idm = 0;              // identity rows (bit m)
   unsigned inr = 0, egN = 0;     // wave-uniform: row m is in the domain; is its last row
   const unsigned egS = (wave == 0 && j0 == 0) ? 1u : 0u;
@@ -621,7 +623,7 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
       const unsigned k = in ? (unsigned)(j * nx + i) : 0u;
       ro[m] = R[k];
       po[m] = Pold[k];
-      xo[m] = X[k];
+      lX[m * NTH] = X[k];
       mo[m] = minv(j, i);
       if (j < ny) inr |= 1u << m;
       if (j == ny - 1) egN |= 1u << m;
@@ -641,10 +643,12 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
   // Frame cells: q0 per thread, counted down so that wave 0, which also waits
   // for the totals, has the outermost; q1 in wave 0 where the frame has more
   // than NTH cells. f: LDS word; bits 16-19 the neighbours it has (E, W, N, S),
-  // 20 identity row, 21-23 within distance 1, 2, 3, 24 received (3 or 4).
+  // 20 identity row, 21-23 within distance 1, 2, 3, 24 received (3 or 4), 25
+  // Jacobi weight 1. Its p is read back from LDS.
   const int q0 = NTH - 1 - tid;
   unsigned f = 0, fk = 0, g = 0, gk = 0;  // fk, gk: byte offsets in the exchange buffers
-  float fr = 0.f, fp = 0.f, fa = 0.f, fc = 0.f, fe = 0.f, fm = 0.f;
+  float fr = 0.f, fa = 0.f, fc = 0.f, fe = 0.f;
+  auto weight = [&]() -> float { return (f & (1u << 25)) ? 1.0f : C.invdf; };
   {
     const float* __restrict__ R = mixed_r(C, KA.parity);
     const float* __restrict__ Pold = mixed_p(C, KA.parity ^ 1);
@@ -662,13 +666,12 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
       if (q0 < F2) f |= 1u << 22;
       if (q0 < F3) f |= 1u << 23;
       if (q0 >= F2) f |= 1u << 24;
-      fm = minv(gj, gi);
+      if (minv(gj, gi) == 1.0f) f |= 1u << 25;
       const unsigned k = (unsigned)(gj * nx + gi);
       fk = 8 * k;
       fr = R[k];
-      fp = Pold[k];
-      lP[f & 0xffffu] = fp;
-      lZ[f & 0xffffu] = fm * fr;
+      lP[f & 0xffffu] = Pold[k];
+      lZ[f & 0xffffu] = weight() * fr;
     }
     if (F4 > NTH && NTH + tid < F4) {
       ca_frame_cell(RH, NTH + tid, row, col);
@@ -754,12 +757,12 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
     return (f & (1u << 20)) ? c : v;
   };
   auto frame_a = [&]() {
-    fa = frame_lap(lP, fp);
-    lMA[f & 0xffffu] = fm * fa;
+    fa = frame_lap(lP, lP[f & 0xffffu]);
+    lMA[f & 0xffffu] = weight() * fa;
   };
   auto frame_ce = [&]() {
-    fc = frame_lap(lMA, fm * fa);
-    fe = frame_lap(lZ, fm * fr);
+    fc = frame_lap(lMA, weight() * fa);
+    fe = frame_lap(lZ, weight() * fr);
   };
   own_a();
   if (f & (1u << 23)) frame_a();
@@ -773,6 +776,9 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
   int n = 0;
   while (true) {
     const unsigned seq = seq0 + 1 + (unsigned)n;
+    // What derives from these is formed where it is used: hoisted out of the
+    // loop it would be spilled, and a reload waits for the stores before it.
+    asm volatile("" : "+v"(f), "+v"(fk), "+v"(g), "+v"(gk), "+v"(e), "+v"(ek), "+v"(watch));
     char* const xb = xch + ((n & 1) ? (size_t)n2 * 8 : 0);
     // The two steps (ca_steps).
 #pragma unroll
@@ -780,7 +786,7 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
       const float z = mo[m] * ro[m], ma = mo[m] * ao[m];
       const float p1 = (z - a0 * ma) + b0 * po[m];
       const float ap1 = (ev[m] - a0 * cv[m]) + b0 * ao[m];
-      xo[m] = (xo[m] + a0 * po[m]) + a1 * p1;
+      lX[m * NTH] = (lX[m * NTH] + a0 * po[m]) + a1 * p1;
       ro[m] = (ro[m] - a0 * ao[m]) - a1 * ap1;
       const float z2 = mo[m] * ro[m];
       po[m] = z2 + b1 * p1;
@@ -788,13 +794,13 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
       own_put(lZ, m, z2);
     }
     if (f & (1u << 22)) {
+      const float fm = weight(), fp = lP[f & 0xffffu];
       const float z = fm * fr, ma = fm * fa;
       const float p1 = (z - a0 * ma) + b0 * fp;
       const float ap1 = (fe - a0 * fc) + b0 * fa;
       fr = (fr - a0 * fa) - a1 * ap1;
       const float z2 = fm * fr;
-      fp = z2 + b1 * p1;
-      lP[f & 0xffffu] = fp;
+      lP[f & 0xffffu] = z2 + b1 * p1;
       lZ[f & 0xffffu] = z2;
     }
     __syncthreads();
@@ -883,9 +889,8 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
       if (all && tid < KCA)
         dev_store((unsigned long long*)(KA.res + kResPart) + ((size_t)((seq + 3) & 3) * KCA + tid) * kResMaxBlk + b, kSent);
       if (f & (1u << 24)) {
-        fp = __uint_as_float((unsigned)(fx >> 32));
         lZ[f & 0xffffu] = __uint_as_float((unsigned)fx);
-        lP[f & 0xffffu] = fp;
+        lP[f & 0xffffu] = __uint_as_float((unsigned)(fx >> 32));
       }
       if (g) {
         lP[g & 0xffffu] = __uint_as_float((unsigned)(gx >> 32));
@@ -947,7 +952,7 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
       const unsigned k = (unsigned)(j * nx + i);
       Rn[k] = ro[m];
       Pn[k] = po[m];
-      X[k] = xo[m];
+      X[k] = lX[m * NTH];
     }
   }
 }
