@@ -89,12 +89,13 @@ struct pf_batch {
   int xd_kinds = 0;      // rounds of those cavities: bit 0 one PCG iteration, bit 1 two
   bool multi = false;    // some cavity has several regions per workgroup
   bool occ2 = false;     // every cavity fits the two-workgroups-per-CU kernel
-  int res_kind = 0;      // rounds with resident solves: 0 none, 1 FP64 (k_round_res64), 2 MIXED (k_round_res32)
+  int res_kind = 0;      // rounds with resident solves: 0 none, 1 FP64 (k_round_res64), 2 MIXED (k_round_res32), 3 MIXED batch (k_round_res32_batch)
   char* dres = nullptr;  // their exchange buffers (KArgs::res), allocated when first used
-  size_t dres_bytes = 0;
+  size_t dres_bytes = 0, res_need = 0;
   bool res_ready = false;  // dres holds its resting values
-  bool res_on = false;     // rounds queued now may run resident solves
+  int res_iters = 0;       // KArgs::res_iters of the rounds queued now; 0: one phase per launch
   int num_cu = 0;
+  int batch_rounds = 64;   // rounds of a solve that a launch of a batch may run (PYFLOW_BATCH_ROUNDS)
   int meet_ticks = 20000;  // KArgs::meet_ticks: 200 us unless PYFLOW_MEET_US says otherwise
   bool s3 = false;       // every cavity runs three PCG iterations per round (k_round_ca3)
   bool tables_dirty = true;
@@ -330,42 +331,46 @@ static bool same_operator(const PfCav& a, const PfCav& b) { return a.op == b.op 
 
 static void drop_graphs(pf_batch* b);
 
-// Batches whose rounds may run a solve by resident workgroups: one cavity
-// (FP64, or MIXED with an FP32 iterate and two PCG iterations per round) with one region of at most 4 tiles per workgroup and no more
-// workgroups than CUs, so that all of them can be on the GPU at once
-// (PYFLOW_RESIDENT=0: never). Results are bitwise the same either way.
+// Batches whose rounds may run a solve by resident workgroups: cavities (one
+// in FP64; MIXED with an FP32 iterate and two PCG iterations per round) with
+// one region of at most 4 tiles per workgroup and no more workgroups each than
+// CUs, so that all of them can be on the GPU at once (PYFLOW_RESIDENT=0:
+// never). Batches of two-tile regions keep the kernel that runs two workgroups
+// per CU. Results are bitwise the same either way.
 static int resident_kind(const pf_batch* b) {
-  if (b->single_slot < 0 || env_switch("PYFLOW_RESIDENT", 1) == 0) return 0;
-  const PfCav& c = b->hcav[b->single_slot];
-  if (c.rpw != 1 || c.tpb > 4 || c.nblk > std::min(b->num_cu, kResMaxBlk)) return 0;
-  if (b->prec == PF_PREC_FP64 && c.nblk == 1 && !c.local) return 0;  // PYFLOW_LOCAL=0: one phase per launch
-  if (b->prec == PF_PREC_FP64) return 1;
-  return c.ca == 1 && !c.xd ? 2 : 0;
+  if (b->total_blocks <= 0 || env_switch("PYFLOW_RESIDENT", 1) == 0) return 0;
+  for (int s = 0; s < b->max_cav; ++s) {
+    if (!b->used[s]) continue;
+    const PfCav& c = b->hcav[s];
+    if (c.rpw != 1 || c.tpb > 4 || c.nblk > std::min(b->num_cu, kResMaxBlk)) return 0;
+    if (b->prec == PF_PREC_MIXED && (c.ca != 1 || c.xd)) return 0;
+    if (b->prec == PF_PREC_FP64 && c.nblk == 1 && !c.local) return 0;  // PYFLOW_LOCAL=0: one phase per launch
+  }
+  if (b->prec == PF_PREC_FP64) return b->single_slot >= 0 ? 1 : 0;
+  return b->single_slot >= 0 ? 2 : (b->occ2 ? 0 : 3);
 }
 
-// Runs (pf_batch_run, pf_batch_launch) let a launch run a whole solve; served
-// batches (pf_batch_advance) keep one phase per launch, so that a chunk of
-// rounds is short whatever the solves need. Puts the exchange buffers into
-// their resting state before the first use.
-static int set_resident(pf_batch* b, bool on) {
-  on = on && b->res_kind != 0;
-  if (on != b->res_on) drop_graphs(b);  // their nodes carry KArgs::res
-  if (on && (!b->res_on || !b->res_ready)) {
-    const PfCav& c = b->hcav[b->single_slot];
-    const size_t need = b->res_kind == 1 ? res64_bytes(c.nblk) : res32_bytes((size_t)c.nx * c.ny);
-    if (b->dres_bytes < need) {
+// Rounds queued from now on may run at most `iters` iterations (FP64) or
+// rounds (MIXED) of a solve in one launch; 0: one phase per launch. Puts the
+// exchange blocks into their resting state before the first use.
+static int set_resident(pf_batch* b, int iters) {
+  if (b->res_kind == 0) iters = 0;
+  if (iters != b->res_iters) drop_graphs(b);  // their nodes carry KArgs::res and res_iters
+  if (iters && (!b->res_iters || !b->res_ready)) {
+    if (b->dres_bytes < b->res_need) {
       if (b->dres) HIPCHK(hipFree(b->dres));
       b->dres = nullptr;
       b->dres_bytes = 0;
       drop_graphs(b);
-      HIPCHK(hipMalloc((void**)&b->dres, need));
-      b->dres_bytes = need;
+      HIPCHK(hipMalloc((void**)&b->dres, b->res_need));
+      b->dres_bytes = b->res_need;
     }
-    HIPCHK(hipMemsetAsync(b->dres, 0xff, b->dres_bytes, b->stream));
-    HIPCHK(hipMemsetAsync(b->dres + kResMeet, 0, 256, b->stream));
+    HIPCHK(hipMemsetAsync(b->dres, 0xff, b->res_need, b->stream));
+    for (int s = 0; s < b->max_cav; ++s)
+      if (b->used[s]) HIPCHK(hipMemsetAsync(b->dres + b->hcav[s].res_off + kResMeet, 0, 256, b->stream));
     b->res_ready = true;
   }
-  b->res_on = on;
+  b->res_iters = iters;
   return PF_OK;
 }
 
@@ -373,11 +378,14 @@ static int sync_tables(pf_batch* b) {
   if (!b->tables_dirty) return PF_OK;
   drop_graphs(b);
   std::vector<int> tiles;  // workgroup -> cavity
+  b->res_need = 0;
   tiles.reserve(b->max_tiles);
   for (int s = 0; s < b->max_cav; ++s) {
     if (!b->used[s]) continue;
     PfCav& c = b->hcav[s];
     c.blk0 = (int)tiles.size();
+    c.res_off = (unsigned)b->res_need;
+    b->res_need += align256(b->prec == PF_PREC_MIXED ? res32_bytes(c.nblk) : res64_bytes(c.nblk));
     for (int t = 0; t < c.nblk; ++t) tiles.push_back(s);
   }
   if ((int64_t)tiles.size() > b->max_tiles) return fail(PF_EINVAL, "batch capacity exceeded");
@@ -481,6 +489,13 @@ static const void* round_fn_u(const pf_batch* b) {
   return b->multi ? round_fn_m<T, U, true>(b) : round_fn_m<T, U, false>(b);
 }
 
+// Iterations (FP64) or rounds (MIXED) a launch may run: whole solves of a single
+// cavity; in a batch the cavities share the CUs, and short turns even out
+// their ends.
+constexpr int kSolveIters = 4096;
+// A cavity of a batch may wait for CUs until others have had their turn.
+constexpr int kBatchMeet = 100;
+
 static const void* res32_fn(int tpb) {
   return tpb == 1 ? (const void*)k_round_res32<1> : tpb == 2 ? (const void*)k_round_res32<2> : (const void*)k_round_res32<4>;
 }
@@ -494,20 +509,19 @@ static RoundLaunch round_launch(const pf_batch* b) {
       const bool one = b->single_slot >= 0;
       L.fn = b->multi ? (one ? (const void*)k_round_ca3<true, true> : (const void*)k_round_ca3<false, true>)
                       : (one ? (const void*)k_round_ca3<true, false> : (const void*)k_round_ca3<false, false>);
-    } else if (b->res_kind == 2 && b->res_on)
-      L.fn = res32_fn(b->hcav[b->single_slot].tpb);
+    } else if (b->res_iters)
+      L.fn = b->res_kind == 2 ? res32_fn(b->hcav[b->single_slot].tpb) : (const void*)k_round_res32_batch;
     else if (b->occ2)
       L.fn = b->single_slot >= 0 ? (const void*)k_round_occ2<true> : (const void*)k_round_occ2<false>;
     else
       L.fn = round_fn_u<float, 2>(b);  // U only shapes the FP64 P/Q loops
     L.lds = (size_t)b->lds_floats * sizeof(float);
-    if (b->res_kind == 2 && b->res_on)
-      L.lds = std::max(L.lds, res32_lds_floats(b->hcav[b->single_slot].tpb) * sizeof(float));
+    if (b->res_iters) L.lds = std::max(L.lds, res32_lds_floats(b->max_tpb) * sizeof(float));
   } else {
     L.fn = b->unroll >= 4 ? round_fn_u<double, 4>(b) : b->unroll == 2 ? round_fn_u<double, 2>(b)
                                                                       : round_fn_u<double, 1>(b);
     L.lds = (size_t)b->lds_floats * sizeof(float);
-    if (b->res_kind == 1 && b->res_on) {
+    if (b->res_iters) {
       L.fn = (const void*)k_round_res64;
       L.lds = std::max(L.lds, res64_lds_doubles(b->hcav[b->single_slot].tpb) * sizeof(double));
     }
@@ -525,8 +539,9 @@ static KArgs round_args(const pf_batch* b, int parity) {
   K.max_cav = b->max_cav;
   K.parity = parity;
   K.slot0 = b->single_slot;
-  K.res = b->res_on ? b->dres : nullptr;
-  K.meet_ticks = b->meet_ticks;
+  K.res = b->res_iters ? b->dres : nullptr;
+  K.res_iters = b->res_iters;
+  K.meet_ticks = b->res_kind == 3 ? kBatchMeet * b->meet_ticks : b->meet_ticks;
   if (b->single_slot >= 0) K.cav0 = b->hcav[b->single_slot];
   return K;
 }
@@ -824,7 +839,8 @@ static int graph_len_of(int rounds) { return rounds <= 0 ? 0 : std::min(1024, st
 
 static int allow_region_lds() {
   const int bytes = std::max({region_lds_floats(8), ca_lds_floats(4), ca3_lds_floats(4), res32_lds_floats(4)}) * (int)sizeof(float);
-  const void* fns[19] = {
+  const void* fns[20] = {
+      (const void*)k_round_res32_batch,
       (const void*)k_round_res32<1>, (const void*)k_round_res32<2>, (const void*)k_round_res32<4>,
       (const void*)k_round_ca3<true, false>, (const void*)k_round_ca3<false, false>,
       (const void*)k_round_ca3<true, true>, (const void*)k_round_ca3<false, true>,
@@ -860,6 +876,7 @@ int pf_batch_create_empty(int precision, int max_cav, int64_t max_tiles, void* s
   // (empty rounds). 1024 against 256 made the 200 steps of the 1024^2 cavity
   // 0.6% faster before that run was tracked. A tracked run (one cavity, several
   // steps) queues at most max_ahead rounds on a prediction (tracked_chunk).
+  b->batch_rounds = std::max(1, std::min(kSolveIters, env_int("PYFLOW_BATCH_ROUNDS", 64)));
   b->meet_ticks = 100 * std::max(0, std::min(1000000, env_switch("PYFLOW_MEET_US", 200)));
   b->max_chunk = std::max<int64_t>(16, env_int("PYFLOW_MAX_CHUNK", 1024));
   b->track = env_switch("PYFLOW_TRACK", 1) != 0;
@@ -1227,7 +1244,7 @@ static int arm(pf_batch* b, int nsteps, const int32_t* active) {
   }
   b->hactive[0] = nact;
   b->hactive[1] = 0;
-  rc = set_resident(b, true);
+  rc = set_resident(b, b->res_kind == 3 ? b->batch_rounds : kSolveIters);
   if (rc) return rc;
   int rc2 = push_scal_all(b);
   if (rc2) return rc2;
@@ -1437,7 +1454,7 @@ int pf_batch_advance(pf_batch* b, int64_t rounds) {
   if (rc) return rc;
   b->serving = true;
   b->obs_slot = -1;
-  rc = set_resident(b, false);
+  rc = set_resident(b, 0);
   if (rc) return rc;
   if (b->total_blocks <= 0) return PF_OK;
   return chunk(b, rounds);

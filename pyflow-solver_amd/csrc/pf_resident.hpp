@@ -26,10 +26,12 @@
 //                 stored by workgroup 0 on kCopies lines (fewer readers per line);
 //   region edges  FP64: one inbox per region side, read by that region only,
 //                 which puts kSent back; two buffers alternate here too.
-//                 MIXED: a region's outer four rows and columns of (r, p), at
-//                 their place in the grid, followed by the region's sequence
-//                 number once the stores have completed; its neighbours wait
-//                 for that number. Two buffers alternate.
+//                 MIXED: z = M r and p of the two rows or columns per side that
+//                 a neighbour's frame needs, packed per region (stores past the
+//                 L2s cost by the line: at 1024^2, cells stored in place in the
+//                 grid took a round from 6.5 to 7.4 us), followed by the region's
+//                 sequence number once the stores have completed; its neighbours
+//                 wait for that number. Two buffers alternate.
 // A sum or cell that equals kSent (a NaN) is stored as another NaN.
 #pragma once
 
@@ -40,19 +42,25 @@ constexpr unsigned long long kOtherNan = 0x7ff8000000000000ull;
 constexpr int kCopies = 8;
 constexpr int kResMaxBlk = 256;           // workgroups of a resident cavity
 constexpr long long kWaitTicks = 1000000000;  // 10 s
-constexpr int kResIters = 4096;           // CG iterations per launch at most
 constexpr double kTinyD = 0x1p-300;
 constexpr unsigned kMeetAbort = 0x10000u;
 
-// Layout of KArgs::res (bytes; every block starts on a 128-byte line).
-constexpr size_t kResMeet = 0;             // arrival words, one per round parity, 128 bytes apart
-constexpr size_t kResBcast = 512;          // FP64: kCopies lines of 16 words
-constexpr size_t kResTotal = 2048;         // MIXED: kCopies lines of 2 KCA words (256 bytes each)
-constexpr size_t kResPart = 4096;          // FP64: 2 x 3 x kResMaxBlk words; MIXED: 4 x KCA x kResMaxBlk words
-constexpr size_t kResFlag = kResPart + 4 * KCA * kResMaxBlk * 8;  // MIXED: a sequence number per workgroup, 128 bytes apart
-constexpr size_t kResData = kResFlag + kResMaxBlk * 128;      // FP64: inboxes [2][nblk][4 sides][64]; MIXED: (r, p) [2][ny][nx]
-__host__ __device__ constexpr size_t res64_bytes(int nblk) { return kResData + (size_t)2 * nblk * 4 * 64 * 8; }
-__host__ __device__ constexpr size_t res32_bytes(size_t cells) { return kResData + 2 * cells * 8; }
+// Exchange block of a cavity, at KArgs::res + PfCav::res_off (bytes; the parts
+// start on 128-byte lines). W = words per partial-sum slot, one a workgroup.
+constexpr size_t kResMeet = 0;      // arrival words, one per round parity, 128 bytes apart
+constexpr size_t kResBcast = 512;   // FP64: kCopies lines of 16 words
+constexpr size_t kResTotal = 2048;  // MIXED: kCopies lines of 2 KCA words (256 bytes each)
+constexpr size_t kResPart = 4096;   // FP64: [2][3][W] words; MIXED: [4][KCA][W]
+__host__ __device__ constexpr size_t res_w(int nblk) { return ((size_t)nblk + 15) / 16 * 16; }
+// FP64: inboxes [2][nblk][4 sides][64] words.
+__host__ __device__ constexpr size_t res64_inbox(int nblk) { return kResPart + 2 * 3 * res_w(nblk) * 8; }
+__host__ __device__ constexpr size_t res64_bytes(int nblk) { return res64_inbox(nblk) + (size_t)2 * nblk * 4 * 64 * 8; }
+// MIXED: a sequence number per workgroup, 128 bytes apart.
+__host__ __device__ constexpr size_t res32_flag(int nblk) { return kResPart + 4 * KCA * res_w(nblk) * 8; }
+// MIXED: edges [2][nblk][4 sides][128] words of (z, p): the two columns (row by
+// row) or rows a neighbour's frame needs from that side.
+__host__ __device__ constexpr size_t res32_edge(int nblk) { return res32_flag(nblk) + (size_t)nblk * 128; }
+__host__ __device__ constexpr size_t res32_bytes(int nblk) { return res32_edge(nblk) + (size_t)2 * nblk * 4 * 128 * 8; }
 enum { SIDE_W = 0, SIDE_E = 1, SIDE_S = 2, SIDE_N = 3 };
 
 constexpr int kResPitch = TX + 3;  // LDS pitch of the FP64 direction: 64 columns, a ring, odd
@@ -94,10 +102,11 @@ __device__ inline bool resident_enter(const KArgs& KA, const PfCav& C, int b, Re
     sh->seq0 = 0;
     sh->tiny[0] = sh->tiny[1] = 0;
     if (nblk > 1) {
-      unsigned* meet = (unsigned*)(KA.res + kResMeet + 128 * KA.parity);
+      char* const res = KA.res + C.res_off;
+      unsigned* meet = (unsigned*)(res + kResMeet + 128 * KA.parity);
       // The last sequence number: FP64 counts broadcasts, MIXED rounds (its flag).
       const unsigned long long* last = (const unsigned long long*)(
-          C.prec == PF_PREC_MIXED ? KA.res + kResFlag + 128 * b : KA.res + kResBcast + 128 * (b & (kCopies - 1)));
+          C.prec == PF_PREC_MIXED ? res + res32_flag(nblk) + 128 * b : res + kResBcast + 128 * (b & (kCopies - 1)));
       const unsigned long long w = dev_load(last);
       sh->seq0 = C.prec == PF_PREC_MIXED ? (unsigned)w : (unsigned)(w >> 32);
       drain_vmem();  // read before arriving: workgroup 0 broadcasts only after every arrival
@@ -127,9 +136,9 @@ __device__ inline bool resident_enter(const KArgs& KA, const PfCav& C, int b, Re
   return sh->go != 0;
 }
 // The previous launch's arrival word, for the launch after this one.
-__device__ inline void resident_clear_meet(const KArgs& KA) {
+__device__ inline void resident_clear_meet(const KArgs& KA, const PfCav& C) {
   if (KA.res != nullptr)
-    __hip_atomic_store((unsigned*)(KA.res + kResMeet + 128 * (KA.parity ^ 1)), 0u, __ATOMIC_RELAXED,
+    __hip_atomic_store((unsigned*)(KA.res + C.res_off + kResMeet + 128 * (KA.parity ^ 1)), 0u, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -194,7 +203,7 @@ __device__ inline double fold_waves(const double* w) {
 }
 
 // The CG iterations of an FP64 solve (phases P and Q of chunk_p / chunk_q and
-// their tails), from a P phase to the end of the solve or kResIters of them.
+// their tails), from a P phase to the end of the solve or KArgs::res_iters of them.
 // A thread keeps x, r, d and q = A d of its M cells in registers; d is also in
 // LDS with a one-cell ring, where the stencil reads it. A region's ring of r is
 // received from its neighbours after every Q, and the ring's d is formed from
@@ -270,7 +279,9 @@ __device__ __attribute__((always_inline)) inline void resident_cg64(const KArgs&
   bool ring = false;
   double rr = 0.0, rd = 0.0, rw = 0.0;
   int ro = 0;
-  unsigned long long* inbox = (unsigned long long*)(KA.res + kResData);
+  char* const res = KA.res + C.res_off;
+  const int W = (int)res_w(nblk);
+  unsigned long long* inbox = (unsigned long long*)(res + res64_inbox(nblk));
   unsigned long long* mine = inbox;
   if (multi && side >= 0 && side < 4) {
     int gi, gj, row, col;
@@ -304,15 +315,15 @@ __device__ __attribute__((always_inline)) inline void resident_cg64(const KArgs&
       inbox + ((size_t)(sendW ? b - 1 : sendE ? b + 1 : 0) * 4 + (sendW ? SIDE_E : SIDE_W)) * 64 + wave;
   unsigned long long* const toS = inbox + ((size_t)(sendS ? b - tiles_x : 0) * 4 + SIDE_N) * 64 + li;
   unsigned long long* const toN = inbox + ((size_t)(sendN ? b + tiles_x : 0) * 4 + SIDE_S) * 64 + li;
-  unsigned long long* const part = (unsigned long long*)(KA.res + kResPart);
-  unsigned long long* const bcast = (unsigned long long*)(KA.res + kResBcast);
+  unsigned long long* const part = (unsigned long long*)(res + kResPart);
+  unsigned long long* const bcast = (unsigned long long*)(res + kResBcast);
   unsigned long long* const line = bcast + 16 * (b & (kCopies - 1));
   unsigned seq = sh.seq0;
   double pq = 0.0, alpha = 0.0, rho_prev = rho, rnorm2 = st.rnorm2;
   bool dead = false;
   int n = 0;
   while (true) {
-    unsigned long long* const pb = part + (n & 1) * 3 * kResMaxBlk;
+    unsigned long long* const pb = part + (n & 1) * 3 * W;
     // P: d = M r (first iteration) or d beta + M r, in registers and LDS.
     const bool first = (it == 0);
     if (tid_flat() == 0) sh.tiny[(n + 1) & 1] = 0;
@@ -462,23 +473,23 @@ __device__ __attribute__((always_inline)) inline void resident_cg64(const KArgs&
       rho = 0.0 + fold_waves(sh.wsum[1]);
       rnorm2 = 0.0 + fold_waves(sh.wsum[2]);
       beta = rho / rho_prev;
-      more = it_total < maxiter && !(sqrt(rnorm2) < atol) && !isnan(rnorm2) && n < kResIters;
+      more = it_total < maxiter && !(sqrt(rnorm2) < atol) && !isnan(rnorm2) && n < KA.res_iters;
     } else {
       if (wave == 0) {
         const double t1 = fold_waves(sh.wsum[1]), t2 = fold_waves(sh.wsum[2]);
-        if (li < 2) dev_store_f64(pb + (1 + li) * kResMaxBlk + b, li ? t2 : t1);
+        if (li < 2) dev_store_f64(pb + (1 + li) * W + b, li ? t2 : t1);
         bool ok = true;
         if (b == 0) {
           double v[4], w[4];
-          ok = words_poll(pb + kResMaxBlk, li, nblk, v);
-          ok = words_poll(pb + 2 * kResMaxBlk, li, nblk, w) && ok;
-          words_reset(pb + kResMaxBlk, li, nblk);
-          words_reset(pb + 2 * kResMaxBlk, li, nblk);
+          ok = words_poll(pb + W, li, nblk, v);
+          ok = words_poll(pb + 2 * W, li, nblk, w) && ok;
+          words_reset(pb + W, li, nblk);
+          words_reset(pb + 2 * W, li, nblk);
           rho_prev = rho;
           rho = fold_words(li, nblk, v);
           rnorm2 = fold_words(li, nblk, w);
           beta = rho / rho_prev;
-          more = it_total < maxiter && !(sqrt(rnorm2) < atol) && !isnan(rnorm2) && n < kResIters;
+          more = it_total < maxiter && !(sqrt(rnorm2) < atol) && !isnan(rnorm2) && n < KA.res_iters;
           const long long u = __double_as_longlong(beta);
           const int wd = li & 3;
           const unsigned pay = wd == 0 ? (unsigned)u : wd == 1 ? (unsigned)(u >> 32) : (more ? 1u : 0u);
@@ -556,7 +567,7 @@ constexpr int kAllToAll = 16;
 
 // The two-iteration PCG rounds of an inner solve of a MIXED cavity (region_ca
 // and tail_ca, FP32 iterate), from a round that runs iterations to the round
-// that ends the inner solve or kResIters rounds. A thread keeps r, p, x of its M
+// that ends the inner solve or KArgs::res_iters rounds. A thread keeps r, p, x of its M
 // cells, and with them a = A p, c = A M a and e = A z: the round forms them of
 // the new basis for its Gram sums, and the next round needs the same values
 // again, so it evaluates three stencils per cell instead of six. p, z and M a
@@ -600,8 +611,8 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
   auto lap = [&](const float* L, float c, int oe, int ow, int on, int os) -> float {
     return __fmul_rn((L[oe] - c) - (c - L[ow]), scx) + __fmul_rn((L[on] - c) - (c - L[os]), scy);
   };
-  const unsigned n2 = (unsigned)(nx * ny);  // at most kResMaxBlk regions: below 2^21 cells
-  char* const xch = KA.res + kResData;
+  char* const res = KA.res + C.res_off;
+  const int W = (int)res_w(nblk);
 
   // Own cells. East and west neighbours by offset (the cell itself where there
   // is none); across the domain's lower and upper edge the wave that holds the
@@ -646,7 +657,25 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
   // 20 identity row, 21-23 within distance 1, 2, 3, 24 received (3 or 4), 25
   // Jacobi weight 1. Its p is read back from LDS.
   const int q0 = NTH - 1 - tid;
-  unsigned f = 0, fk = 0, g = 0, gk = 0;  // fk, gk: byte offsets in the exchange buffers
+  unsigned f = 0, fk = 0, g = 0, gk = 0;  // fk, gk: byte offsets of received cells among the edges
+  // Byte offset of the cell at (row, col) of the frame, distance 3 or 4, among
+  // the edges: its region, and which of that region's sides has it.
+  auto edge_of = [&](int row, int col) -> unsigned {
+    const int dy = row < 4 ? row - 4 : (row >= RH + 4 ? row - RH - 3 : 0);  // signed distance from the region
+    const int dx = col < 4 ? col - 4 : (col >= TX + 4 ? col - TX - 3 : 0);
+    const int reg = b + (dx > 0 ? 1 : dx < 0 ? -1 : 0) + (dy > 0 ? tiles_x : dy < 0 ? -tiles_x : 0);
+    int side, w;
+    if (dx <= -3 || dx >= 3) {  // its east columns TX-4, TX-3 or its west columns 2, 3
+      side = dx < 0 ? SIDE_E : SIDE_W;
+      const int r = dy == 0 ? row - 4 : dy < 0 ? RH + dy : dy - 1;
+      w = 2 * r + (dx < 0 ? dx + 4 : dx - 3);
+    } else {
+      side = dy < 0 ? SIDE_N : SIDE_S;
+      const int q = dx == 0 ? col - 4 : dx < 0 ? TX + dx : dx - 1;
+      w = (dy < 0 ? dy + 4 : dy - 3) * TX + q;
+    }
+    return 8u * (unsigned)((reg * 4 + side) * 128 + w);
+  };
   float fr = 0.f, fa = 0.f, fc = 0.f, fe = 0.f;
   auto weight = [&]() -> float { return (f & (1u << 25)) ? 1.0f : C.invdf; };
   {
@@ -668,7 +697,7 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
       if (q0 >= F2) f |= 1u << 24;
       if (minv(gj, gi) == 1.0f) f |= 1u << 25;
       const unsigned k = (unsigned)(gj * nx + gi);
-      fk = 8 * k;
+      if (q0 >= F2) fk = edge_of(row, col);
       fr = R[k];
       lP[f & 0xffffu] = Pold[k];
       lZ[f & 0xffffu] = weight() * fr;
@@ -680,33 +709,22 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
       if (gi >= 0 && gi < nx && gj >= 0 && gj < ny) {
         g = (unsigned)(row * HQ + col) | (1u << 24);
         const unsigned k = (unsigned)(gj * nx + gi);
-        gk = 8 * k;
+        gk = edge_of(row, col);
         lP[g & 0xffffu] = Pold[k];
         lZ[g & 0xffffu] = minv(gj, gi) * R[k];
       }
     }
   }
-  // The cell this thread publishes after every round, if any (e: LDS word, bit
-  // 24 set). A neighbour's frame at distances 3 and 4 needs the region's rows
-  // and columns 2 and 3 from each side that has a neighbour.
-  unsigned e = 0, ek = 0;
-  {
-    int row = -1, col = 0;
-    if (tid < 4 * TX) {
-      const int t = tid / TX;
-      row = t < 2 ? 2 + t : RH - 6 + t;
-      col = tid % TX;
-    } else if (tid < 4 * TX + 4 * (RH - 4)) {
-      const int q = tid - 4 * TX, t = q / (RH - 4), k = q % (RH - 4);
-      col = t < 2 ? 2 + t : TX - 6 + t;
-      row = k < 2 ? k : (k < RH - 6 ? k + 2 : k + 4);
-    }
-    const bool byrow = ((row == 2 || row == 3) && j0 > 0) || ((row == RH - 4 || row == RH - 3) && j0 + RH < ny);
-    const bool bycol = ((col == 2 || col == 3) && rx > 0) || ((col == TX - 4 || col == TX - 3) && i0 + TX < nx);
-    if (row >= 0 && (byrow || bycol) && row < rows && i0 + col < nx) {
-      e = (unsigned)((row + 4) * HQ + col + 4) | (1u << 24);
-      ek = 8 * (unsigned)((j0 + row) * nx + i0 + col);
-    }
+  // The word of the edges this thread publishes after every round, if any (e:
+  // LDS word of its cell, bit 24 set): 128 threads per side that has a neighbour.
+  unsigned e = 0;
+  const unsigned ek = 8u * (unsigned)(b * 512 + tid);
+  if (tid < 512) {
+    const int side = tid >> 7, w = tid & 127;
+    const int row = side < 2 ? w >> 1 : (side == SIDE_S ? 2 : RH - 4) + (w >> 6);
+    const int col = side < 2 ? (side == SIDE_W ? 2 : TX - 4) + (w & 1) : w & 63;
+    const bool to = side == SIDE_W ? rx > 0 : side == SIDE_E ? i0 + TX < nx : side == SIDE_S ? j0 > 0 : j0 + RH < ny;
+    if (to && row < rows && i0 + col < nx) e = (unsigned)((row + 4) * HQ + col + 4) | (1u << 24);
   }
   // The neighbour whose sequence number lane 0..7 of wave 15 watches, else the
   // region itself.
@@ -778,8 +796,8 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
     const unsigned seq = seq0 + 1 + (unsigned)n;
     // What derives from these is formed where it is used: hoisted out of the
     // loop it would be spilled, and a reload waits for the stores before it.
-    asm volatile("" : "+v"(f), "+v"(fk), "+v"(g), "+v"(gk), "+v"(e), "+v"(ek), "+v"(watch));
-    char* const xb = xch + ((n & 1) ? (size_t)n2 * 8 : 0);
+    asm volatile("" : "+v"(f), "+v"(fk), "+v"(g), "+v"(gk), "+v"(e), "+v"(watch));
+    char* const xb = res + res32_edge(nblk) + ((n & 1) ? (size_t)nblk * 4096 : 0);
     // The two steps (ca_steps).
 #pragma unroll
     for (int m = 0; m < M; ++m) {
@@ -839,17 +857,17 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
     wave_partials_ca(acc, [&](int k, double v) { sh.wtot[k][wave] = v; });
     drain_vmem();  // the published cells are in memory before the barrier, so before the flag
     __syncthreads();
-    unsigned long long* const pb = (unsigned long long*)(KA.res + kResPart) + (size_t)(seq & 3) * KCA * kResMaxBlk;
+    unsigned long long* const pb = (unsigned long long*)(res + kResPart) + (size_t)(seq & 3) * KCA * W;
     if (tid < KCA) {
       const double t = fold_waves(sh.wtot[tid]);
       if (multi)
-        dev_store_f64(pb + tid * kResMaxBlk + b, t);
+        dev_store_f64(pb + tid * W + b, t);
       else
         sh.tot[tid] = 0.0 + t;
     }
     if (multi) {
       if (wave == NWAVE - 1) {
-        unsigned long long* const flags = (unsigned long long*)(KA.res + kResFlag);
+        unsigned long long* const flags = (unsigned long long*)(res + res32_flag(nblk));
         if (li == 0) dev_store(flags + 16 * b, (unsigned long long)seq);
         const long long t0 = wall_clock64();
         while (true) {
@@ -869,16 +887,16 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
         bool ok = true;
         for (int k = slot; k < KCA; k += all ? KCA : 8 * nown) {
           double v[4];
-          ok = words_poll(pb + k * kResMaxBlk, li, nblk, v) && ok;
+          ok = words_poll(pb + k * W, li, nblk, v) && ok;
           const double t = fold_words(li, nblk, v);
           if (all) {
             if (li == 0) sh.tot[k] = t;
           } else {
             const unsigned long long u = (unsigned long long)__double_as_longlong(t);
             const unsigned pay = (li & 1) ? (unsigned)(u >> 32) : (unsigned)u;
-            unsigned long long* const total = (unsigned long long*)(KA.res + kResTotal);
+            unsigned long long* const total = (unsigned long long*)(res + kResTotal);
             if (li < 2 * kCopies) dev_store(total + 32 * (li >> 1) + 2 * k + (li & 1), pay | ((unsigned long long)seq << 32));
-            words_reset(pb + k * kResMaxBlk, li, nblk);
+            words_reset(pb + k * W, li, nblk);
           }
         }
         if (!ok && li == 0) sh.dead = 1;
@@ -887,14 +905,14 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
       // the launch before, if this is the first) back to kSent: every workgroup has
       // read them, since all have stored this round's.
       if (all && tid < KCA)
-        dev_store((unsigned long long*)(KA.res + kResPart) + ((size_t)((seq + 3) & 3) * KCA + tid) * kResMaxBlk + b, kSent);
+        dev_store((unsigned long long*)(res + kResPart) + ((size_t)((seq + 3) & 3) * KCA + tid) * W + b, kSent);
       if (f & (1u << 24)) {
         lZ[f & 0xffffu] = __uint_as_float((unsigned)fx);
         lP[f & 0xffffu] = __uint_as_float((unsigned)(fx >> 32));
       }
       if (g) {
-        lP[g & 0xffffu] = __uint_as_float((unsigned)(gx >> 32));
         lZ[g & 0xffffu] = __uint_as_float((unsigned)gx);
+        lP[g & 0xffffu] = __uint_as_float((unsigned)(gx >> 32));
       }
     }
     __syncthreads();
@@ -904,7 +922,7 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
     if (wave == 0) {
       if (!all) {
         unsigned pay;
-        const unsigned long long* const line = (const unsigned long long*)(KA.res + kResTotal) + 32 * (b & (kCopies - 1));
+        const unsigned long long* const line = (const unsigned long long*)(res + kResTotal) + 32 * (b & (kCopies - 1));
         const bool ok = bcast_wait(line, li, 2 * KCA, seq, pay);
         if (li < 2 * KCA) ((unsigned*)sh.tot)[li] = pay;
         if (!ok && li == 0) sh.dead = 1;
@@ -917,7 +935,7 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
         sh.coef[2] = (float)r.a1;
         sh.coef[3] = (float)r.b1;
         sh.inc = r.n;
-        sh.go = (r.next == 0 && n + 1 < kResIters) ? 1 : 0;
+        sh.go = (r.next == 0 && n + 1 < KA.res_iters) ? 1 : 0;
         if (b == 0 && sh.go == 0) {
           st.it += it_total - st.it_total;
           st.it_run += it_total - st.it_total;

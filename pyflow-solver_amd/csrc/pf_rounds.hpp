@@ -114,6 +114,7 @@ struct PfCav {
   double* part;                                 // [2][NPS][nblk]: slot k of workgroup b at k*nblk + b
   float* y;                                     // MIXED: deflation vector (nullptr in FP64)
   int defl;  // MIXED, pinned operator: Galerkin correction along y = A^-1 1 after each solve
+  unsigned res_off;  // its exchange block for resident solves, at KArgs::res + res_off
   int local;  // FP64, one region: the CG iterations of a solve run inside one round (local_cg)
 };
 
@@ -2203,7 +2204,8 @@ struct KArgs {
   int parity;
   int slot0;   // SINGLE: the cavity's slot
   int meet_ticks;  // resident solves: how long workgroups wait for each other to start (100 MHz clock)
-  char* res;   // exchange buffers of the resident solves (pf_resident.hpp); nullptr: one phase per launch
+  char* res;   // exchange blocks of the resident solves (pf_resident.hpp); nullptr: one phase per launch
+  int res_iters;  // resident solves: FP64 iterations, MIXED rounds, per launch at most
   PfCav cav0;  // SINGLE: the cavity's descriptor
 };
 
@@ -2908,7 +2910,7 @@ __global__ __launch_bounds__(NTH) void k_round_res64(const KArgs KA) {
   const PfCav* Cg = KA.cavs + KA.slot0;
   const int lg = blockIdx.x - C.blk0;
   const int b = ((C.blk0 & 7) == 0 && (C.nblk & 7) == 0) ? (lg & 7) * (C.nblk >> 3) + (lg >> 3) : lg;
-  if (b == 0 && tid_flat() == 0) resident_clear_meet(KA);
+  if (b == 0 && tid_flat() == 0) resident_clear_meet(KA, C);
   round_body<double, 2, 0, false, false, true>(KA, C, Cg, KA.slot0, b, st, sm, tot, lds_dyn, &rsh);
 }
 
@@ -2926,8 +2928,30 @@ __global__ __launch_bounds__(NTH) void k_round_res32(const KArgs KA) {
   const PfCav* Cg = KA.cavs + KA.slot0;
   const int lg = blockIdx.x - C.blk0;
   const int b = ((C.blk0 & 7) == 0 && (C.nblk & 7) == 0) ? (lg & 7) * (C.nblk >> 3) + (lg >> 3) : lg;
-  if (b == 0 && tid_flat() == 0) resident_clear_meet(KA);
+  if (b == 0 && tid_flat() == 0) resident_clear_meet(KA, C);
   round_body_ca<M, false, false, 3, true>(KA, C, Cg, KA.slot0, b, st, sm, tot, lds_dyn, &rsh);
+}
+
+// Batches of such cavities. A launch that holds more workgroups than the GPU
+// dispatches them in order, so the workgroups of the first unfinished cavity
+// are always the next to get a CU, whichever cavities wait for theirs.
+__global__ __launch_bounds__(NTH) void k_round_res32_batch(const KArgs KA) {
+  __shared__ PfScal st;
+  __shared__ double sm[NWAVE][NPS];
+  __shared__ double tot[NPS];
+  __shared__ ResShared rsh;
+  extern __shared__ float lds_dyn[];  // the largest of the cavities' ca_lds_floats and res32_lds_floats
+  const int c = KA.blk_cav[blockIdx.x];
+  if (c < 0) return;
+  const PfCav& C = KA.cavs[c];
+  const int lg = blockIdx.x - C.blk0;
+  const int b = ((C.blk0 & 7) == 0 && (C.nblk & 7) == 0) ? (lg & 7) * (C.nblk >> 3) + (lg >> 3) : lg;
+  if (b == 0 && tid_flat() == 0) resident_clear_meet(KA, C);
+  switch (C.tpb) {
+    case 1: round_body_ca<1, false, false, 3, true>(KA, C, KA.cavs + c, c, b, st, sm, tot, lds_dyn, &rsh); break;
+    case 2: round_body_ca<2, false, false, 3, true>(KA, C, KA.cavs + c, c, b, st, sm, tot, lds_dyn, &rsh); break;
+    default: round_body_ca<4, false, false, 3, true>(KA, C, KA.cavs + c, c, b, st, sm, tot, lds_dyn, &rsh); break;
+  }
 }
 
 // Batches whose cavities all run three PCG iterations per round (PfCav::ca
