@@ -94,8 +94,9 @@ struct pf_batch {
   size_t dres_bytes = 0, res_need = 0;
   bool res_ready = false;  // dres holds its resting values
   int res_iters = 0;       // KArgs::res_iters of the rounds queued now; 0: one phase per launch
+  bool res_turns = false;  // they run k_round_res32_batch, PCG turns and other phases by kBatchCycle
   int num_cu = 0;
-  int batch_rounds = 64;   // rounds of a solve that a launch of a batch may run (PYFLOW_BATCH_ROUNDS)
+  int batch_rounds = 128;  // rounds of a solve that a launch of a batch may run (PYFLOW_BATCH_ROUNDS)
   int meet_ticks = 20000;  // KArgs::meet_ticks: 200 us unless PYFLOW_MEET_US says otherwise
   bool s3 = false;       // every cavity runs three PCG iterations per round (k_round_ca3)
   bool tables_dirty = true;
@@ -353,9 +354,10 @@ static int resident_kind(const pf_batch* b) {
 // Rounds queued from now on may run at most `iters` iterations (FP64) or
 // rounds (MIXED) of a solve in one launch; 0: one phase per launch. Puts the
 // exchange blocks into their resting state before the first use.
-static int set_resident(pf_batch* b, int iters) {
+static int set_resident(pf_batch* b, int iters, bool turns) {
   if (b->res_kind == 0) iters = 0;
-  if (iters != b->res_iters) drop_graphs(b);  // their nodes carry KArgs::res and res_iters
+  turns = turns && iters > 0;
+  if (iters != b->res_iters || turns != b->res_turns) drop_graphs(b);  // their nodes carry KArgs::res and res_iters
   if (iters && (!b->res_iters || !b->res_ready)) {
     if (b->dres_bytes < b->res_need) {
       if (b->dres) HIPCHK(hipFree(b->dres));
@@ -371,6 +373,7 @@ static int set_resident(pf_batch* b, int iters) {
     b->res_ready = true;
   }
   b->res_iters = iters;
+  b->res_turns = turns;
   return PF_OK;
 }
 
@@ -493,6 +496,7 @@ static const void* round_fn_u(const pf_batch* b) {
 // cavity; in a batch the cavities share the CUs, and short turns even out
 // their ends.
 constexpr int kSolveIters = 4096;
+constexpr int kServeRounds = 64;
 // A cavity of a batch may wait for CUs until others have had their turn.
 constexpr int kBatchMeet = 100;
 
@@ -510,7 +514,7 @@ static RoundLaunch round_launch(const pf_batch* b) {
       L.fn = b->multi ? (one ? (const void*)k_round_ca3<true, true> : (const void*)k_round_ca3<false, true>)
                       : (one ? (const void*)k_round_ca3<true, false> : (const void*)k_round_ca3<false, false>);
     } else if (b->res_iters)
-      L.fn = b->res_kind == 2 ? res32_fn(b->hcav[b->single_slot].tpb) : (const void*)k_round_res32_batch;
+      L.fn = b->res_turns ? (const void*)k_round_res32_batch : res32_fn(b->hcav[b->single_slot].tpb);
     else if (b->occ2)
       L.fn = b->single_slot >= 0 ? (const void*)k_round_occ2<true> : (const void*)k_round_occ2<false>;
     else
@@ -529,7 +533,14 @@ static RoundLaunch round_launch(const pf_batch* b) {
   return L;
 }
 
-static KArgs round_args(const pf_batch* b, int parity) {
+// Round k of a batch with resident solves: every kBatchCycle-th launch lets each
+// cavity run its PCG, the others only the phases between (a cavity in its PCG
+// is passed over). Otherwise a cavity with a dozen short phases ahead would
+// take one per launch, each as long as its neighbours' turns.
+constexpr int kBatchCycle = 8;
+
+static KArgs round_args(const pf_batch* b, int parity, int64_t k, int cycle = 0) {
+  if (cycle <= 0 || cycle > kBatchCycle) cycle = kBatchCycle;
   KArgs K;
   std::memset(&K, 0, sizeof(K));
   K.cavs = b->dcav;
@@ -540,8 +551,8 @@ static KArgs round_args(const pf_batch* b, int parity) {
   K.parity = parity;
   K.slot0 = b->single_slot;
   K.res = b->res_iters ? b->dres : nullptr;
-  K.res_iters = b->res_iters;
-  K.meet_ticks = b->res_kind == 3 ? kBatchMeet * b->meet_ticks : b->meet_ticks;
+  K.res_iters = (b->res_turns && k % cycle != cycle - 1) ? -1 : b->res_iters;
+  K.meet_ticks = b->res_turns ? kBatchMeet * b->meet_ticks : b->meet_ticks;
   if (b->single_slot >= 0) K.cav0 = b->hcav[b->single_slot];
   return K;
 }
@@ -550,7 +561,7 @@ static hipError_t launch_rounds_direct(pf_batch* b, int64_t n) {
   if (b->total_blocks <= 0 || n <= 0) return hipSuccess;
   const RoundLaunch L = round_launch(b);
   for (int64_t r = 0; r < n; ++r) {
-    KArgs K = round_args(b, (int)(b->round & 1));
+    KArgs K = round_args(b, (int)(b->round & 1), b->round);
     void* args[] = {&K};
     const hipError_t e = hipLaunchKernel(L.fn, L.grid, L.blk, args, L.lds, b->stream);
     if (e != hipSuccess) return e;
@@ -578,7 +589,7 @@ static int build_graph(pf_batch* b, int par) {
   hipGraphNode_t prev = nullptr;
   hipError_t e = hipSuccess;
   for (int k = 0; k < b->graph_len && e == hipSuccess; ++k) {
-    KArgs K = round_args(b, par ^ (k & 1));
+    KArgs K = round_args(b, par ^ (k & 1), k, b->graph_len);
     void* args[] = {&K};
     hipKernelNodeParams np;
     std::memset(&np, 0, sizeof(np));
@@ -618,6 +629,27 @@ static int launch_rounds(pf_batch* b, int64_t n) {
   }
   HIPCHK(launch_rounds_direct(b, n));
   b->rounds += n;
+  return PF_OK;
+}
+
+// Rounds of a served batch with resident solves: of every 64 (or what is left),
+// up to seven are launches for the other phases, and the rest are one launch in
+// which every cavity in its PCG runs that many rounds of it.
+static int launch_served(pf_batch* b, int64_t n) {
+  const RoundLaunch L = round_launch(b);
+  while (n > 0) {
+    const int turn = (int)std::min<int64_t>(n, kServeRounds);
+    const int others = std::min(kBatchCycle - 1, turn - 1);
+    for (int k = 0; k <= others; ++k) {
+      KArgs K = round_args(b, (int)(b->round & 1), 0);
+      K.res_iters = k < others ? -1 : turn - others;
+      void* args[] = {&K};
+      HIPCHK(hipLaunchKernel(L.fn, L.grid, L.blk, args, L.lds, b->stream));
+      b->round += 1;
+      b->rounds += 1;
+    }
+    n -= turn;
+  }
   return PF_OK;
 }
 
@@ -876,7 +908,7 @@ int pf_batch_create_empty(int precision, int max_cav, int64_t max_tiles, void* s
   // (empty rounds). 1024 against 256 made the 200 steps of the 1024^2 cavity
   // 0.6% faster before that run was tracked. A tracked run (one cavity, several
   // steps) queues at most max_ahead rounds on a prediction (tracked_chunk).
-  b->batch_rounds = std::max(1, std::min(kSolveIters, env_int("PYFLOW_BATCH_ROUNDS", 64)));
+  b->batch_rounds = std::max(1, std::min(kSolveIters, env_int("PYFLOW_BATCH_ROUNDS", 128)));
   b->meet_ticks = 100 * std::max(0, std::min(1000000, env_switch("PYFLOW_MEET_US", 200)));
   b->max_chunk = std::max<int64_t>(16, env_int("PYFLOW_MAX_CHUNK", 1024));
   b->track = env_switch("PYFLOW_TRACK", 1) != 0;
@@ -1227,6 +1259,7 @@ static int arm(pf_batch* b, int nsteps, const int32_t* active) {
     sc.step_round = 0;
     sc.step_len = 0;
     sc.dsetup = 0;
+    sc.flip = 0;
     if (c.mode == PF_MODE_STEP) {
       sc.phase = PH_STATS;
       sc.steps_left = nsteps;
@@ -1244,7 +1277,7 @@ static int arm(pf_batch* b, int nsteps, const int32_t* active) {
   }
   b->hactive[0] = nact;
   b->hactive[1] = 0;
-  rc = set_resident(b, b->res_kind == 3 ? b->batch_rounds : kSolveIters);
+  rc = set_resident(b, b->res_kind == 3 ? b->batch_rounds : kSolveIters, b->res_kind == 3);
   if (rc) return rc;
   int rc2 = push_scal_all(b);
   if (rc2) return rc2;
@@ -1258,7 +1291,7 @@ static int arm(pf_batch* b, int nsteps, const int32_t* active) {
 static int chunk(pf_batch* b, int64_t n) {
   b->scal_fresh = false;
   if (b->timing) HIPCHK(hipEventRecord(b->ev_t0, b->stream));
-  const int rc = launch_rounds(b, n);
+  const int rc = (b->serving && b->res_turns) ? launch_served(b, n) : launch_rounds(b, n);
   if (rc) return rc;
   HIPCHK(hipGetLastError());
   if (b->timing) {
@@ -1428,6 +1461,7 @@ int pf_batch_start(pf_batch* b, int slot, int nsteps) {
   sc.step_round = 0;
   sc.step_len = 0;
   sc.dsetup = 0;
+  sc.flip = 0;
   if (c.mode == PF_MODE_STEP) {
     sc.phase = PH_STATS;
     sc.steps_left = nsteps;
@@ -1454,7 +1488,8 @@ int pf_batch_advance(pf_batch* b, int64_t rounds) {
   if (rc) return rc;
   b->serving = true;
   b->obs_slot = -1;
-  rc = set_resident(b, 0);
+  // Served MIXED cavities run their PCG in turns too (launch_served).
+  rc = set_resident(b, b->res_kind >= 2 ? kServeRounds : 0, true);
   if (rc) return rc;
   if (b->total_blocks <= 0) return PF_OK;
   return chunk(b, rounds);

@@ -84,9 +84,10 @@ struct ResShared {
   double val[2];          // FP64: alpha, beta
   float coef[4];          // MIXED: alpha_k, beta_k, alpha_k+1, beta_k+1
   double tot[KCA];        // MIXED: totals of the round
-  double wtot[KCA][NWAVE];  // MIXED: wave totals
+  double wtot[KCA][NWAVE + 2];  // MIXED: wave totals (rows 144 bytes apart: 14 lanes read a row each)
   double wsum[3][NWAVE];  // wave totals: P, and the two of Q
   unsigned seq0;        // sequence number of the last broadcast before this launch
+  unsigned nbseq;  // MIXED: round whose edges all neighbours have published
   int go, dead, inc;
   int tiny[2];  // some d of the region or its ring is a tiny number, by iteration parity
 };
@@ -109,6 +110,7 @@ __device__ inline bool resident_enter(const KArgs& KA, const PfCav& C, int b, Re
           C.prec == PF_PREC_MIXED ? res + res32_flag(nblk) + 128 * b : res + kResBcast + 128 * (b & (kCopies - 1)));
       const unsigned long long w = dev_load(last);
       sh->seq0 = C.prec == PF_PREC_MIXED ? (unsigned)w : (unsigned)(w >> 32);
+      sh->nbseq = sh->seq0;
       drain_vmem();  // read before arriving: workgroup 0 broadcasts only after every arrival
       const long long t0 = wall_clock64();
       unsigned cur = __hip_atomic_fetch_add(meet, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
@@ -612,6 +614,7 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
     return __fmul_rn((L[oe] - c) - (c - L[ow]), scx) + __fmul_rn((L[on] - c) - (c - L[os]), scy);
   };
   char* const res = KA.res + C.res_off;
+  const int par = KA.parity ^ st.flip;  // of the r and p buffers
   const int W = (int)res_w(nblk);
 
   // Own cells. East and west neighbours by offset (the cell itself where there
@@ -624,8 +627,8 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
   unsigned inr = 0, egN = 0;     // wave-uniform: row m is in the domain; is its last row
   const unsigned egS = (wave == 0 && j0 == 0) ? 1u : 0u;
   {
-    const float* __restrict__ R = mixed_r(C, KA.parity);
-    const float* __restrict__ Pold = mixed_p(C, KA.parity ^ 1);
+    const float* __restrict__ R = mixed_r(C, par);
+    const float* __restrict__ Pold = mixed_p(C, par ^ 1);
     const float* __restrict__ X = (const float*)C.x;
 #pragma unroll
     for (int m = 0; m < M; ++m) {
@@ -679,8 +682,8 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
   float fr = 0.f, fa = 0.f, fc = 0.f, fe = 0.f;
   auto weight = [&]() -> float { return (f & (1u << 25)) ? 1.0f : C.invdf; };
   {
-    const float* __restrict__ R = mixed_r(C, KA.parity);
-    const float* __restrict__ Pold = mixed_p(C, KA.parity ^ 1);
+    const float* __restrict__ R = mixed_r(C, par);
+    const float* __restrict__ Pold = mixed_p(C, par ^ 1);
     int row = 0, col = 0;
     if (q0 < F4) ca_frame_cell(RH, q0, row, col);
     int gj = j0 + row - 4, gi = i0 + col - 4;
@@ -718,7 +721,6 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
   // The word of the edges this thread publishes after every round, if any (e:
   // LDS word of its cell, bit 24 set): 128 threads per side that has a neighbour.
   unsigned e = 0;
-  const unsigned ek = 8u * (unsigned)(b * 512 + tid);
   if (tid < 512) {
     const int side = tid >> 7, w = tid & 127;
     const int row = side < 2 ? w >> 1 : (side == SIDE_S ? 2 : RH - 4) + (w >> 6);
@@ -796,7 +798,8 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
     const unsigned seq = seq0 + 1 + (unsigned)n;
     // What derives from these is formed where it is used: hoisted out of the
     // loop it would be spilled, and a reload waits for the stores before it.
-    asm volatile("" : "+v"(f), "+v"(fk), "+v"(g), "+v"(gk), "+v"(e), "+v"(watch));
+    int lv = li;
+    asm volatile("" : "+v"(f), "+v"(fk), "+v"(g), "+v"(gk), "+v"(e), "+v"(watch), "+v"(lv));
     char* const xb = res + res32_edge(nblk) + ((n & 1) ? (size_t)nblk * 4096 : 0);
     // The two steps (ca_steps).
 #pragma unroll
@@ -824,7 +827,7 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
     __syncthreads();
     if (e) {
       const unsigned o = e & 0xffffu;
-      dev_store((unsigned long long*)(xb + ek),
+      dev_store((unsigned long long*)(xb + 8u * (unsigned)(b * 512 + wave * TX + lv)),
                 (unsigned long long)__float_as_uint(lZ[o]) | ((unsigned long long)__float_as_uint(lP[o]) << 32));
     }
     own_a();
@@ -832,38 +835,47 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
     __syncthreads();
     // c, e and the Gram sums of the new basis (pass 5 of region_ca).
     double acc[NP] = {0.0, 0.0, 0.0, 0.0};
+    auto gram = [&](int m) {
+      const double p2 = po[m], z2 = mo[m] * ro[m], r2 = ro[m], a2 = ao[m];
+      const double ma2 = mo[m] * ao[m], c2 = cv[m], mc2 = mo[m] * cv[m], e2 = ev[m], me2 = mo[m] * ev[m];
+      acc[0] = __fma_rn(p2, a2, acc[0]);
+      acc[1] = __fma_rn(p2, c2, acc[1]);
+      acc[2] = __fma_rn(p2, e2, acc[2]);
+      acc[3] = __fma_rn(a2, ma2, acc[3]);
+      acc[4] = __fma_rn(a2, mc2, acc[4]);
+      acc[5] = __fma_rn(a2, z2, acc[5]);
+      acc[6] = __fma_rn(a2, me2, acc[6]);
+      acc[7] = __fma_rn(c2, mc2, acc[7]);
+      acc[8] = __fma_rn(c2, z2, acc[8]);
+      acc[9] = __fma_rn(c2, me2, acc[9]);
+      acc[10] = __fma_rn(r2, z2, acc[10]);
+      acc[11] = __fma_rn(z2, e2, acc[11]);
+      acc[12] = __fma_rn(e2, me2, acc[12]);
+      acc[13] = __fma_rn(r2, r2, acc[13]);
+    };
+    if (full) {
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-      own_ce(m);
-      if (full || (((inr >> m) & 1u) && i < nx)) {
-        const double p2 = po[m], z2 = mo[m] * ro[m], r2 = ro[m], a2 = ao[m];
-        const double ma2 = mo[m] * ao[m], c2 = cv[m], mc2 = mo[m] * cv[m], e2 = ev[m], me2 = mo[m] * ev[m];
-        acc[0] = __fma_rn(p2, a2, acc[0]);
-        acc[1] = __fma_rn(p2, c2, acc[1]);
-        acc[2] = __fma_rn(p2, e2, acc[2]);
-        acc[3] = __fma_rn(a2, ma2, acc[3]);
-        acc[4] = __fma_rn(a2, mc2, acc[4]);
-        acc[5] = __fma_rn(a2, z2, acc[5]);
-        acc[6] = __fma_rn(a2, me2, acc[6]);
-        acc[7] = __fma_rn(c2, mc2, acc[7]);
-        acc[8] = __fma_rn(c2, z2, acc[8]);
-        acc[9] = __fma_rn(c2, me2, acc[9]);
-        acc[10] = __fma_rn(r2, z2, acc[10]);
-        acc[11] = __fma_rn(z2, e2, acc[11]);
-        acc[12] = __fma_rn(e2, me2, acc[12]);
-        acc[13] = __fma_rn(r2, r2, acc[13]);
+      for (int m = 0; m < M; ++m) {
+        own_ce(m);
+        gram(m);
+      }
+    } else {
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        own_ce(m);
+        if (((inr >> m) & 1u) && i < nx) gram(m);
       }
     }
     wave_partials_ca(acc, [&](int k, double v) { sh.wtot[k][wave] = v; });
     drain_vmem();  // the published cells are in memory before the barrier, so before the flag
     __syncthreads();
     unsigned long long* const pb = (unsigned long long*)(res + kResPart) + (size_t)(seq & 3) * KCA * W;
-    if (tid < KCA) {
-      const double t = fold_waves(sh.wtot[tid]);
+    if (wave == 0 && lv < KCA) {
+      const double t = fold_waves(sh.wtot[lv]);
       if (multi)
-        dev_store_f64(pb + tid * W + b, t);
+        dev_store_f64(pb + lv * W + b, t);
       else
-        sh.tot[tid] = 0.0 + t;
+        sh.tot[lv] = 0.0 + t;
     }
     if (multi) {
       if (wave == NWAVE - 1) {
@@ -878,8 +890,14 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
             break;
           }
         }
+        if (li == 0) __hip_atomic_store(&sh.nbseq, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
-      __syncthreads();  // the neighbours' cells are in memory
+      // Waves that receive wait for that (wave 15's wait is bounded).
+      if (__any(((f | g) >> 24) & 1u)) {
+        while (__hip_atomic_load(&sh.nbseq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != seq)
+          __builtin_amdgcn_s_sleep(1);
+        asm volatile("" ::: "memory");
+      }
       unsigned long long fx = 0, gx = 0;
       if (f & (1u << 24)) fx = dev_load((const unsigned long long*)(xb + fk));
       if (g) gx = dev_load((const unsigned long long*)(xb + gk));
@@ -887,16 +905,16 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
         bool ok = true;
         for (int k = slot; k < KCA; k += all ? KCA : 8 * nown) {
           double v[4];
-          ok = words_poll(pb + k * W, li, nblk, v) && ok;
-          const double t = fold_words(li, nblk, v);
+          ok = words_poll(pb + k * W, lv, nblk, v) && ok;
+          const double t = fold_words(lv, nblk, v);
           if (all) {
             if (li == 0) sh.tot[k] = t;
           } else {
             const unsigned long long u = (unsigned long long)__double_as_longlong(t);
-            const unsigned pay = (li & 1) ? (unsigned)(u >> 32) : (unsigned)u;
+            const unsigned pay = (lv & 1) ? (unsigned)(u >> 32) : (unsigned)u;
             unsigned long long* const total = (unsigned long long*)(res + kResTotal);
-            if (li < 2 * kCopies) dev_store(total + 32 * (li >> 1) + 2 * k + (li & 1), pay | ((unsigned long long)seq << 32));
-            words_reset(pb + k * W, li, nblk);
+            if (lv < 2 * kCopies) dev_store(total + 32 * (lv >> 1) + 2 * k + (lv & 1), pay | ((unsigned long long)seq << 32));
+            words_reset(pb + k * W, lv, nblk);
           }
         }
         if (!ok && li == 0) sh.dead = 1;
@@ -904,8 +922,8 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
       // Each workgroup puts its own words of the round before (the last one of
       // the launch before, if this is the first) back to kSent: every workgroup has
       // read them, since all have stored this round's.
-      if (all && tid < KCA)
-        dev_store((unsigned long long*)(res + kResPart) + ((size_t)((seq + 3) & 3) * KCA + tid) * W + b, kSent);
+      if (all && wave == 0 && lv < KCA)
+        dev_store((unsigned long long*)(res + kResPart) + ((size_t)((seq + 3) & 3) * KCA + lv) * W + b, kSent);
       if (f & (1u << 24)) {
         lZ[f & 0xffffu] = __uint_as_float((unsigned)fx);
         lP[f & 0xffffu] = __uint_as_float((unsigned)(fx >> 32));
@@ -923,8 +941,8 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
       if (!all) {
         unsigned pay;
         const unsigned long long* const line = (const unsigned long long*)(res + kResTotal) + 32 * (b & (kCopies - 1));
-        const bool ok = bcast_wait(line, li, 2 * KCA, seq, pay);
-        if (li < 2 * KCA) ((unsigned*)sh.tot)[li] = pay;
+        const bool ok = bcast_wait(line, lv, 2 * KCA, seq, pay);
+        if (lv < 2 * KCA) ((unsigned*)sh.tot)[lv] = pay;
         if (!ok && li == 0) sh.dead = 1;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       }
@@ -960,8 +978,8 @@ __device__ __attribute__((always_inline)) inline void resident_ca(const KArgs& K
     return;
   }
   // Leave the vectors as a round of this parity leaves them.
-  float* __restrict__ Rn = mixed_r(C, KA.parity ^ 1);
-  float* __restrict__ Pn = mixed_p(C, KA.parity);
+  float* __restrict__ Rn = mixed_r(C, par ^ 1);
+  float* __restrict__ Pn = mixed_p(C, par);
   float* __restrict__ X = (float*)C.x;
 #pragma unroll
   for (int m = 0; m < M; ++m) {

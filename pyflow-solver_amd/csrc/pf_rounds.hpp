@@ -130,7 +130,8 @@ struct PfScal {
   int dready;      // y holds the deflation vector of this cavity's operator
   int step_round;  // rounds_run when the last projection step ended
   int step_len;    // rounds_run of the last projection step (the host sizes its chunks with it)
-  int pad_[2];
+  int flip;        // MIXED: the PCG's r and p buffers are one parity off the round's (launches passed over)
+  int pad_;
   double dden;     // y.A y of the stored y
   double dcoef;    // Galerkin coefficient of the finished solve
   double dt_prev, dt, cfl_now, umax, vmax, hist[5], div_before;
@@ -385,37 +386,30 @@ __device__ __attribute__((always_inline)) inline CaTail tail_ca_steps(const doub
   if (r.next) return r;
   const double w01 = t[0], w02 = t[1], w04 = t[2], w11 = t[3], w12 = t[4], w13 = t[5], w14 = t[6];
   const double w22 = t[7], w23 = t[8], w24 = t[9], w33 = t[10], w34 = t[11], w44 = t[12];
-  double a0 = w33 / w01;
-  double b0 = 0.0, a1 = 0.0, b1 = 0.0;
-  int n = 1;
+  // Without branches (every wave of the grid waits for this chain of four
+  // divisions): all of it is formed, then the cases are selected.
   // alpha < 0 is legitimate: the Dirichlet operator (+lap) is negative
   // definite. gamma = r.M r > 0 whatever the sign of A.
-  if (a0 == 0.0 || !isfinite(a0)) {
-    // No usable step (only reachable with corrupted input): count one
-    // iteration and restart the direction at p = M r.
-    a0 = 0.0;
-  } else {
-    const double g1 = w33 - 2.0 * a0 * w13 + a0 * a0 * w11;
-    b0 = g1 / w33;
-    const double pap = (w34 - a0 * w23 + b0 * w13) + (-a0 * w14 + a0 * a0 * w12 - a0 * b0 * w11) +
-                       (b0 * w04 - a0 * b0 * w02 + b0 * b0 * w01);
-    const double a1c = g1 / pap;
-    if (maxiter - it_total >= 2 && g1 > 0.0 && pap != 0.0 && isfinite(a1c)) {
-      a1 = a1c;
-      n = 2;
-      const double k1 = -(a0 + a1 * b0), k2 = a1 * a0, k4 = -a1;
-      const double g2 = w33 + k1 * k1 * w11 + k2 * k2 * w22 + k4 * k4 * w44 +
-                        2.0 * (k1 * w13 + k2 * w23 + k4 * w34 + k1 * k2 * w12 + k1 * k4 * w14 + k2 * k4 * w24);
-      b1 = g2 / g1;
-      if (!isfinite(b1)) b1 = 0.0;
-    }
-    if (!isfinite(b0)) b0 = 0.0;
-  }
-  r.a0 = a0;
-  r.b0 = b0;
-  r.a1 = a1;
-  r.b1 = b1;
-  r.n = n;
+  const double a0 = w33 / w01;
+  const double g1 = w33 - 2.0 * a0 * w13 + a0 * a0 * w11;
+  const double b0 = g1 / w33;
+  const double pap = (w34 - a0 * w23 + b0 * w13) + (-a0 * w14 + a0 * a0 * w12 - a0 * b0 * w11) +
+                     (b0 * w04 - a0 * b0 * w02 + b0 * b0 * w01);
+  const double a1 = g1 / pap;
+  const double k1 = -(a0 + a1 * b0), k2 = a1 * a0, k4 = -a1;
+  const double g2 = w33 + k1 * k1 * w11 + k2 * k2 * w22 + k4 * k4 * w44 +
+                    2.0 * (k1 * w13 + k2 * w23 + k4 * w34 + k1 * k2 * w12 + k1 * k4 * w14 + k2 * k4 * w24);
+  const double b1 = g2 / g1;
+  // No usable step (only reachable with corrupted input): count one iteration
+  // and restart the direction at p = M r. One iteration, too, where the budget
+  // has room for one or the second step breaks down.
+  const bool one = a0 != 0.0 && isfinite(a0);
+  const bool two = one && maxiter - it_total >= 2 && g1 > 0.0 && pap != 0.0 && isfinite(a1);
+  r.a0 = one ? a0 : 0.0;
+  r.b0 = one && isfinite(b0) ? b0 : 0.0;
+  r.a1 = two ? a1 : 0.0;
+  r.b1 = two && isfinite(b1) ? b1 : 0.0;
+  r.n = two ? 2 : 1;
   return r;
 }
 // The state after the tail of a round that left the totals t and ran S.ca_inc
@@ -2205,7 +2199,7 @@ struct KArgs {
   int slot0;   // SINGLE: the cavity's slot
   int meet_ticks;  // resident solves: how long workgroups wait for each other to start (100 MHz clock)
   char* res;   // exchange blocks of the resident solves (pf_resident.hpp); nullptr: one phase per launch
-  int res_iters;  // resident solves: FP64 iterations, MIXED rounds, per launch at most
+  int res_iters;  // resident solves: FP64 iterations, MIXED rounds, per launch at most; -1: a launch for the other phases
   PfCav cav0;  // SINGLE: the cavity's descriptor
 };
 
@@ -2651,15 +2645,23 @@ __device__ __attribute__((always_inline)) inline void round_body_ca(const KArgs&
     return;
   }
   if constexpr (RES) {
-    if (phase == PH_CG && st.ca_inc > 0 && resident_enter(KA, C, b, rsh)) {
-      resident_ca<M>(KA, C, st, *rsh, lds, b);
-      if (b == 0) {
-        __syncthreads();
-        if (tid == 0 && !st.dsetup) st.rounds_run += 1;
-        __syncthreads();
-        if (tid < NW32) dst[tid] = ((const uint32_t*)&st)[tid];
+    if (phase == PH_CG && st.ca_inc > 0) {
+      // A launch for the other phases of a batch (KArgs::res_iters < 0) passes
+      // over a cavity in its PCG; the round parity moves on, its buffers do not.
+      const bool pass = KA.res_iters < 0;
+      if (pass || resident_enter(KA, C, b, rsh)) {
+        if (!pass) resident_ca<M>(KA, C, st, *rsh, lds, b);
+        if (b == 0) {
+          __syncthreads();
+          if (tid == 0) {
+            if (!st.dsetup) st.rounds_run += 1;
+            st.flip = (pass && st.phase == PH_CG) ? st.flip ^ 1 : (st.phase == PH_CG ? st.flip : 0);
+          }
+          __syncthreads();
+          if (tid < NW32) dst[tid] = ((const uint32_t*)&st)[tid];
+        }
+        return;
       }
-      return;
     }
   }
   PhaseArgs A;
@@ -2669,7 +2671,7 @@ __device__ __attribute__((always_inline)) inline void round_body_ca(const KArgs&
   A.alpha = st.alpha;
   A.it = st.it;
   A.x_is_b = st.x_is_b;
-  A.par = parity;
+  A.par = (phase == PH_CG) ? parity ^ st.flip : parity;
   A.x0 = (phase == PH_DEFL_B) ? st.dcoef : 0.0;  // FIN reads x[0] in round_cold
   A.cx = C.cxf;
   A.cy = C.cyf;
@@ -2702,6 +2704,7 @@ __device__ __attribute__((always_inline)) inline void round_body_ca(const KArgs&
     __syncthreads();
     if (tid == 0) {
       st.pending = phase;
+      if (phase != PH_CG) st.flip = 0;
       if (!st.dsetup) st.rounds_run += 1;
     }
     __syncthreads();

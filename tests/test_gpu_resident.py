@@ -216,3 +216,38 @@ def test_concurrent_streams_bitwise(precision):
     for r in both:
         for x in r:
             assert np.array_equal(x, alone[0][0])
+
+
+@pytest.mark.parametrize("sizes", [
+    [(512, 512), (449, 300), (64, 64), (33, 40), (512, 384), (200, 640), (96, 96), (512, 448)],  # more workgroups than CUs
+    [(130, 97), (16, 16), (65, 17)],
+])
+def test_batch_bitwise(sizes):
+    """A batch whose cavities run their PCG in turns, against one phase per
+    launch for all: three steps, then one more."""
+    from pyflow._device import DeviceBatch, cavity_params
+    out = []
+    for resident in ("0", "1"):
+        ps = [cavity_params(nx, ny, dx=1.0, dy=1.0, scheme="quick", lid_velocity=1.0, Re=300.0 * (k + 1), lin_tol=1e-6,
+                            lin_maxiter=3000) for k, (nx, ny) in enumerate(sizes)]
+        print(f"[resident] batch of {len(sizes)} resident={resident}", flush=True)
+        old = os.environ.get("PYFLOW_RESIDENT")
+        os.environ["PYFLOW_RESIDENT"] = resident
+        try:
+            b = DeviceBatch(ps, "mixed")
+            d = [b.run(n) for n in (3, 1)]
+        finally:
+            if old is None:
+                del os.environ["PYFLOW_RESIDENT"]
+            else:
+                os.environ["PYFLOW_RESIDENT"] = old
+        f = []
+        for k, (nx, ny) in enumerate(sizes):
+            a = [np.zeros((ny + 2, nx + 2)) for _ in range(3)]
+            b.download(k, *a)
+            f += a
+        b.close()
+        out.append((f, [(x[k].rp_iterations_run, x[k].rp_residual, x[k].continuity) for x in d for k in range(len(sizes))]))
+    for x, y in zip(out[0][0], out[1][0]):
+        assert np.array_equal(x, y)
+    assert out[0][1] == out[1][1]
