@@ -88,6 +88,8 @@ struct pf_batch {
   bool any_xd = false;   // some cavity keeps its PCG iterate in FP64
   int xd_kinds = 0;      // rounds of those cavities: bit 0 one PCG iteration, bit 1 two
   bool multi = false;    // some cavity has several regions per workgroup
+  bool march = false;    // every cavity runs marching rounds (k_round_march)
+  bool marchers = false; // some do
   bool occ2 = false;     // every cavity fits the two-workgroups-per-CU kernel
   int res_kind = 0;      // rounds with resident solves: 0 none, 1 FP64 (k_round_res64), 2 MIXED (k_round_res32), 3 MIXED batch (k_round_res32_batch)
   char* dres = nullptr;  // their exchange buffers (KArgs::res), allocated when first used
@@ -205,6 +207,33 @@ static size_t cavity_bytes(int prec, const pf_cavity_params* p) {
   return s;
 }
 
+// Strips of a marching round (pf_march.hpp): cavities with several regions per
+// workgroup that run two PCG iterations per round. As few strips as cover the
+// columns, of even width; as many segments as there are waves for them. More
+// waves hide more latency, but shorten the segments, whose 8 extra rows are
+// half (1040^2) to a sixth (4096^2) of their work: 16, 12, 8 waves of a
+// workgroup take 24.6, 22.6, 22.7 us a round at 1040^2, 33.3, 31.7, 32.6 at
+// 1535^2 and 126.4, 126.2, 133.9 at 4096^2 (solves of 400 iterations, start
+// included). On regions they take 25.9, 45.3 and 184.
+// With an FP64 iterate, the last bits of the step lengths reach the FP64
+// residual of the next refinement pass, so that another order of the sums
+// moves the solution within its tolerance (p of a 2048^2 step by 4e-8). Up to
+// 2048^2, where regions take 48.9 us and strips 43.0, those cavities keep
+// regions and their bits; above it strips gain far more (98 -> 64 us at 2560^2).
+constexpr int kMarchWaves = 12;
+constexpr int64_t kMarchXdCells = 2048 * 2048;
+static void plan_march(PfCav& c) {
+  c.mstrips = c.msegs = c.mown = c.mlen = c.mwaves = 0;
+  if (c.prec != PF_PREC_MIXED || c.ca != 1 || c.rpw < 2) return;
+  if (c.xd && (int64_t)c.nx * c.ny <= kMarchXdCells) return;
+  c.mstrips = (c.nx + kStripOwn - 1) / kStripOwn;
+  c.mown = ((c.nx + c.mstrips - 1) / c.mstrips + 1) & ~1;
+  c.mwaves = kMarchWaves;
+  const int segs = std::max(1, c.nblk * c.mwaves / c.mstrips);
+  c.mlen = (c.ny + segs - 1) / segs;
+  c.msegs = (c.ny + c.mlen - 1) / c.mlen;
+}
+
 // MIXED: two PCG iterations per round (regions of up to 4 tiles; their
 // 4-cell frames fit in LDS), with an FP32 or an FP64 iterate. Default on;
 // PYFLOW_CA=0 (FP32 iterate) or PYFLOW_CA_XD=0 (FP64 iterate) turns it off,
@@ -219,12 +248,14 @@ static void choose_ca(PfCav& c, int prec, int pcg_per_round) {
     c.ca = 2;
   else
     c.ca = (prec == PF_PREC_MIXED && c.tpb <= 4 && s >= 2) ? 1 : 0;
+  plan_march(c);
 }
 
 // Dynamic LDS of a cavity's round: the float32 PCG region's staging, or in
 // FP64 the direction array of the in-round CG (local_cg).
 static int lds_floats_of(const PfCav& c) {
   if (c.prec != PF_PREC_MIXED) return c.local ? 2 * c.nx * c.ny : 0;
+  if (c.mstrips) return 0;
   return c.ca == 2 ? ca3_lds_floats(c.tpb) : (c.ca ? ca_lds_floats(c.tpb) : region_lds_floats(c.tpb));
 }
 
@@ -405,6 +436,8 @@ static int sync_tables(pf_batch* b) {
   b->any_xd = false;
   b->xd_kinds = 0;
   b->multi = false;
+  b->march = nused > 0;
+  b->marchers = false;
   b->occ2 = (b->prec == PF_PREC_MIXED) && env_switch("PYFLOW_OCC2", 1) != 0;
   int n3 = 0;
   for (int s = 0; s < b->max_cav; ++s)
@@ -422,6 +455,8 @@ static int sync_tables(pf_batch* b) {
       const PfCav& c = b->hcav[s];
       b->occ2 = b->occ2 && c.ca == 1 && !c.xd && c.tpb <= 2 && c.rpw == 1;
       b->multi = b->multi || b->hcav[s].rpw > 1;
+      b->march = b->march && c.mstrips > 0;
+      b->marchers = b->marchers || c.mstrips > 0;
     }
   b->res_kind = resident_kind(b);
   b->res_ready = false;
@@ -478,6 +513,9 @@ static const void* round_fn_m(const pf_batch* b) {
   // FP64-iterate cavities are large (a round takes 100+ us): their descriptor
   // is read from the table (the by-value copy would only add register
   // pressure to the bigger kernel).
+  if constexpr (MULTI && sizeof(T) == sizeof(float)) {
+    if (b->marchers) return (const void*)k_round<T, U, false, 7, true>;
+  }
   if (sizeof(T) == sizeof(float) && b->any_xd) {
     if (b->xd_kinds == 2) return (const void*)k_round<T, U, false, 2, MULTI>;
     if (b->xd_kinds == 3) return (const void*)k_round<T, U, false, 3, MULTI>;
@@ -515,6 +553,8 @@ static RoundLaunch round_launch(const pf_batch* b) {
                       : (one ? (const void*)k_round_ca3<true, false> : (const void*)k_round_ca3<false, false>);
     } else if (b->res_iters)
       L.fn = b->res_turns ? (const void*)k_round_res32_batch : res32_fn(b->hcav[b->single_slot].tpb);
+    else if (b->march)
+      L.fn = b->single_slot >= 0 ? (const void*)k_round_march<true> : (const void*)k_round_march<false>;
     else if (b->occ2)
       L.fn = b->single_slot >= 0 ? (const void*)k_round_occ2<true> : (const void*)k_round_occ2<false>;
     else
@@ -871,7 +911,8 @@ static int graph_len_of(int rounds) { return rounds <= 0 ? 0 : std::min(1024, st
 
 static int allow_region_lds() {
   const int bytes = std::max({region_lds_floats(8), ca_lds_floats(4), ca3_lds_floats(4), res32_lds_floats(4)}) * (int)sizeof(float);
-  const void* fns[20] = {
+  const void* fns[21] = {
+      (const void*)k_round<float, 2, false, 7, true>,
       (const void*)k_round_res32_batch,
       (const void*)k_round_res32<1>, (const void*)k_round_res32<2>, (const void*)k_round_res32<4>,
       (const void*)k_round_ca3<true, false>, (const void*)k_round_ca3<false, false>,
@@ -1667,6 +1708,7 @@ int pf_solve_noalloc(int precision, const pf_cavity_params* params, const double
   tb.any_xd = c.xd != 0;
   tb.xd_kinds = c.xd ? (c.ca ? 2 : 1) : 0;
   tb.multi = c.rpw > 1;
+  tb.march = tb.marchers = c.mstrips > 0;
   tb.s3 = c.ca == 2;
   tb.occ2 = (precision == PF_PREC_MIXED) && env_switch("PYFLOW_OCC2", 1) != 0 && c.ca == 1 && !c.xd && c.tpb <= 2 &&
             c.rpw == 1;

@@ -130,6 +130,9 @@ struct PfCav {
   int defl;  // MIXED, pinned operator: Galerkin correction along y = A^-1 1 after each solve
   unsigned res_off;  // its exchange block for resident solves, at KArgs::res + res_off
   int local;  // FP64, one region: the CG iterations of a solve run inside one round (local_cg)
+  // Marching rounds (pf_march.hpp): strips and segments, their own columns and
+  // rows at most, waves of a workgroup that march; mstrips 0: region_ca.
+  int mstrips, msegs, mown, mlen, mwaves;
 };
 
 // Scalar state of one cavity; two copies (round parity) per cavity.
@@ -2400,6 +2403,7 @@ __device__ __attribute__((noinline)) void local_cg(const PfCav* __restrict__ Cg,
 }
 
 }  // namespace pf
+#include "pf_march.hpp"
 #include "pf_resident.hpp"
 namespace pf {
 
@@ -2590,7 +2594,7 @@ __device__ __attribute__((always_inline)) inline void round_body(const KArgs& KA
 // partials are folded by one wave per slot: wave w sums slot w of every
 // workgroup (per lane: increasing workgroup index; then the DPP tree), so all
 // fourteen slots of the PCG round fold in parallel; thread 63 runs the tail.
-// RES: a round that runs iterations may run the rest of its inner solve in this
+// M: the region's height in tiles; 0: a marching round (march_ca). RES: a round that runs iterations may run the rest of its inner solve in this
 // launch (resident_ca).
 template <int M, bool MULTI, bool XD, int V = 0, bool RES = false>
 __device__ __attribute__((always_inline)) inline void round_body_ca(const KArgs& KA, const PfCav& C, const PfCav* Cg, int c,
@@ -2702,9 +2706,13 @@ __device__ __attribute__((always_inline)) inline void round_body_ca(const KArgs&
   // The partials' address is formed after the region loop (from the
   // descriptor again), which keeps it out of the loop's registers.
   if (__builtin_expect(phase == PH_CG, 1)) {
-    for (int r = r0; r < r1; ++r) {
-      if (r > r0) __syncthreads();  // the previous region's LDS reads are done
-      region_ca<M, XD>(C, A, r, acc, lds);
+    if constexpr (M == 0) {
+      march_ca<XD>(C, A, b, acc);
+    } else {
+      for (int r = r0; r < r1; ++r) {
+        if (r > r0) __syncthreads();  // the previous region's LDS reads are done
+        region_ca<M, XD>(C, A, r, acc, lds);
+      }
     }
     block_partials_ca(acc, sm, C.part + (size_t)parity * C.nblk * NPS + b, C.nblk);
   } else {
@@ -2879,7 +2887,12 @@ __global__ __launch_bounds__(NTH) void k_round(const KArgs KA) {
   const int lg = g - C.blk0;
   const int b = ((C.blk0 & 7) == 0 && (C.nblk & 7) == 0) ? (lg & 7) * (C.nblk >> 3) + (lg >> 3) : lg;
   if constexpr (sizeof(T) == sizeof(float)) {
-    if ((XDK & 2) && C.xd && C.ca) {
+    if ((XDK & 4) && C.mstrips) {
+      if (C.xd)
+        round_body_ca<0, false, true>(KA, C, Cg, c, b, st, sm, tot, lds_dyn);
+      else
+        round_body_ca<0, false, false>(KA, C, Cg, c, b, st, sm, tot, lds_dyn);
+    } else if ((XDK & 2) && C.xd && C.ca) {
       switch (C.tpb) {
         case 1: round_body_ca<1, MULTI, true>(KA, C, Cg, c, b, st, sm, tot, lds_dyn); break;
         case 2: round_body_ca<2, MULTI, true>(KA, C, Cg, c, b, st, sm, tot, lds_dyn); break;
@@ -2892,11 +2905,11 @@ __global__ __launch_bounds__(NTH) void k_round(const KArgs KA) {
         case 4: round_body<T, U, 4, true, MULTI>(KA, C, Cg, c, b, st, sm, tot, lds_dyn); break;
         default: round_body<T, U, 8, true, MULTI>(KA, C, Cg, c, b, st, sm, tot, lds_dyn); break;
       }
-    } else if (C.ca) {
+    } else if (C.ca) {  // one region per workgroup: with more, an FP32 iterate marches
       switch (C.tpb) {
-        case 1: round_body_ca<1, MULTI, false>(KA, C, Cg, c, b, st, sm, tot, lds_dyn); break;
-        case 2: round_body_ca<2, MULTI, false>(KA, C, Cg, c, b, st, sm, tot, lds_dyn); break;
-        default: round_body_ca<4, MULTI, false>(KA, C, Cg, c, b, st, sm, tot, lds_dyn); break;
+        case 1: round_body_ca<1, false, false>(KA, C, Cg, c, b, st, sm, tot, lds_dyn); break;
+        case 2: round_body_ca<2, false, false>(KA, C, Cg, c, b, st, sm, tot, lds_dyn); break;
+        default: round_body_ca<4, false, false>(KA, C, Cg, c, b, st, sm, tot, lds_dyn); break;
       }
     } else {
       switch (C.tpb) {
@@ -2909,6 +2922,23 @@ __global__ __launch_bounds__(NTH) void k_round(const KArgs KA) {
   } else {
     round_body<T, U, 0, false, MULTI>(KA, C, Cg, c, b, st, sm, tot, lds_dyn);
   }
+}
+
+// Batches whose cavities all march (PfCav::mstrips).
+template <bool SINGLE>
+__global__ __launch_bounds__(NTH) void k_round_march(const KArgs KA) {
+  __shared__ PfScal st;
+  __shared__ double sm[NWAVE][NPS];
+  __shared__ double tot[NPS];
+  const int c = SINGLE ? KA.slot0 : KA.blk_cav[blockIdx.x];
+  if (c < 0) return;
+  const PfCav& C = KA.cavs[c];
+  const int lg = blockIdx.x - C.blk0;
+  const int b = ((C.blk0 & 7) == 0 && (C.nblk & 7) == 0) ? (lg & 7) * (C.nblk >> 3) + (lg >> 3) : lg;
+  if (C.xd)
+    round_body_ca<0, false, true, 4>(KA, C, &C, c, b, st, sm, tot, nullptr);
+  else
+    round_body_ca<0, false, false, 4>(KA, C, &C, c, b, st, sm, tot, nullptr);
 }
 
 // Single FP64 cavities whose workgroups all fit on the GPU at once: the rounds
