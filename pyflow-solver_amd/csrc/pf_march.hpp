@@ -41,15 +41,6 @@ __device__ __attribute__((always_inline)) inline float lane_down(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xF, 0xF, true));  // wave_shr:1
 }
 
-// Values that are the same in every lane, moved to scalar registers.
-__device__ __attribute__((always_inline)) inline float uniform(float v) {
-  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-__device__ __attribute__((always_inline)) inline double uniform(double v) {
-  const long long u = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readfirstlane((int)(u & 0xffffffffll)), hi = __builtin_amdgcn_readfirstlane((int)(u >> 32));
-  return __longlong_as_double((long long)(unsigned)lo | ((long long)hi << 32));
-}
 // One strip segment. EDGE: it reads or owns cells on or beyond the domain's
 // boundary, where neighbours are missing, weights are 1, rows may be
 // identity rows, and loads go cell by cell to clamped places.

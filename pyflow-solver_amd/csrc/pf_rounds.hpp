@@ -41,6 +41,16 @@ __device__ __attribute__((always_inline)) inline PF_GLOBAL V* uniform(V* p) {
   return (PF_GLOBAL V*)((unsigned long long)lo | ((unsigned long long)hi << 32));
 }
 
+// Values that are the same in every lane, moved to scalar registers.
+__device__ __attribute__((always_inline)) inline float uniform(float v) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+__device__ __attribute__((always_inline)) inline double uniform(double v) {
+  const long long u = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readfirstlane((int)(u & 0xffffffffll)), hi = __builtin_amdgcn_readfirstlane((int)(u >> 32));
+  return __longlong_as_double((long long)(unsigned)lo | ((long long)hi << 32));
+}
+
 // Stores of the PCG rounds' r, p and x: streaming (non-temporal) by default;
 // build with -DPF_STREAM_STORES=0 for ordinary stores.
 #ifndef PF_STREAM_STORES
@@ -1450,19 +1460,55 @@ __device__ __attribute__((always_inline)) inline CaCell ca_steps(const PhaseArgs
   return o;
 }
 
+// The frame cells of a thread: LDS row and column (row << 8 | col) of frame
+// cell tid, and of cell tid + NTH where the frame has more than NTH (loads
+// only); ~0 where there is none. The same for every region of a workgroup.
+struct CaFrame {
+  unsigned a, b;
+};
+template <int M>
+__device__ __attribute__((always_inline)) inline CaFrame ca_frame() {
+  constexpr int F4 = ca_frame_cells(TY * M, 4);
+  const int tid = tid_flat();
+  CaFrame f{~0u, ~0u};
+  int row, col;
+  if (tid < F4) {
+    ca_frame_cell(TY * M, tid, row, col);
+    f.a = (unsigned)(row << 8 | col);
+  }
+  if (F4 > NTH && tid + NTH < F4) {
+    ca_frame_cell(TY * M, tid + NTH, row, col);
+    f.b = (unsigned)(row << 8 | col);
+  }
+  return f;
+}
+
 // XD: the iterate is the FP64 x64 (x64 += alpha_k p_k + alpha_k+1 p_k+1 in
 // FP64), as in the one-iteration FP64-iterate round.
+//
+// The vector instructions bound it (16 waves a CU), with the load latency of
+// each region of a workgroup ahead of them; loading the next region under pass
+// 5 gained nothing (45.7 against 46.2 us at 2048^2, and 4% lost where a
+// workgroup has one region). What tells the domain's
+// edges apart is kept out of the cells' code: a cell without an east or west
+// neighbour reads itself there (its difference is +0, as the reflective
+// stencil has it), the wave with the domain's first or last row keeps a copy of
+// it in the LDS row beyond, identity rows and rows beyond the domain are
+// wave-uniform branches. Against ghost and identity codes per cell: 48.9 -> 46.2
+// us a round at 2048^2 (FP64 iterate, solve start included), a step on one
+// phase per launch at 1024^2 19.0 -> 17.5 ms, 64 cavities of 96^2 two to a CU
+// 10.1 -> 9.2 ms, 128 of 32^2 to 512^2 at 16 workgroups each 609 -> 542 ms.
 template <int M, bool XD>
-__device__ __attribute__((always_inline)) inline void region_ca(const PfCav& C, const PhaseArgs& A, int r, double* acc,
+__device__ __attribute__((always_inline)) inline void region_ca(const PfCav& C, const PhaseArgs& A, int r,
+                                                                const CaFrame& F, double* acc,
                                                                 float* __restrict__ lds) {
-  const int nx = C.nx, ny = C.ny;
+  const int nx = __builtin_amdgcn_readfirstlane(C.nx), ny = __builtin_amdgcn_readfirstlane(C.ny);
   constexpr int RH = TY * M;
-  constexpr int NR = RH + 8;
+  constexpr int NR = RH + 8, TP = TY * HQ;
   constexpr int F1 = ca_frame_cells(RH, 1), F2 = ca_frame_cells(RH, 2), F3 = ca_frame_cells(RH, 3);
-  constexpr int F4 = ca_frame_cells(RH, 4);
-  constexpr int NS = (F4 + NTH - 1) / NTH;  // frame slots per thread; slots past the first are loads only
-  static_assert(F3 <= NTH, "one thread per frame cell within distance 3");
+  static_assert(F3 <= NTH && ca_frame_cells(RH, 4) <= 2 * NTH, "one thread per frame cell within distance 3");
   static_assert(NR * HQ * 5 == ca_lds_floats(M), "LDS layout");
+  static_assert(NR < 256 && HQ < 256, "CaFrame packs rows and columns");
   float* __restrict__ lP = lds;                 // p_k
   float* __restrict__ lZ = lds + NR * HQ;       // z_k = M r_k
   float* __restrict__ lMA = lds + 2 * NR * HQ;  // M A p_k, then M A p_k+2
@@ -1472,199 +1518,205 @@ __device__ __attribute__((always_inline)) inline void region_ca(const PfCav& C, 
   // write r[q^1], p[q]. The basis-only round runs the round after PINIT /
   // OUTER_B, which wrote r[q^1]: it reads r there, leaves r and x as they
   // are (the next round reads r[q^1] again) and writes p = M r to p[q].
-  const bool init = A.ca_init != 0;
+  const bool init = __builtin_amdgcn_readfirstlane(A.ca_init) != 0;
   using XT = std::conditional_t<XD, double, float>;
   const PF_GLOBAL float* __restrict__ R = uniform(mixed_r(C, init ? (A.par ^ 1) : A.par));
   const PF_GLOBAL float* __restrict__ Pold = uniform(mixed_p(C, A.par ^ 1));
   PF_GLOBAL float* __restrict__ Rn = uniform(mixed_r(C, A.par ^ 1));
   PF_GLOBAL float* __restrict__ Pn = uniform(mixed_p(C, A.par));
   PF_GLOBAL XT* __restrict__ X = uniform((XT*)(XD ? (void*)C.x64 : C.x));
-  const int li = threadIdx.x, lj = threadIdx.y;
-  const int tid = lj * TX + li;
-  const int i0 = (r % C.tiles_x) * TX;
-  const int j0 = (r / C.tiles_x) * RH;
+  const int li = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);  // = the row within a tile
+  const int tid = wave * TX + li;
+  const int ry = __builtin_amdgcn_readfirstlane(r / C.tiles_x), rx = __builtin_amdgcn_readfirstlane(r % C.tiles_x);
+  const int i0 = rx * TX;
+  const int j0 = ry * RH;
   const int i = i0 + li;
-  // Operator without boundary tests. A cell on the domain boundary also
-  // writes its value into the LDS ghost across that boundary, so the missing
-  // neighbour's difference (e - c etc.) is exactly +0, as the reflective
-  // stencil drops it (lap5_fast); the operator's sign is folded into
-  // 1/dx^2, 1/dy^2 (round-to-nearest is sign-symmetric). Identity rows (the
-  // pinned cell; the Dirichlet boundary) return the cell's value. Cells
-  // outside the domain are never written and never read.
-  const bool pinned = (C.op == 0);
-  const float scx = pinned ? -A.cx : A.cx, scy = pinned ? -A.cy : A.cy;
-  // Cell code: LDS offsets of the (at most two) ghosts the cell writes, the
-  // cell's own offset standing in for a missing one; bit 30 marks a cell with
-  // a ghost (only those write the copies: 4096^2 207 instead of 217 us per
-  // round, 1024^2 13.7 instead of 14.2 us), bit 31 an identity row.
-  auto code_of = [&](int gj, int gi, int row, int col) -> unsigned {
-    const int o = row * HQ + col;
-    int g1 = o, g2 = o;
-    if (gi == nx - 1 && col + 1 < HQ) g1 = o + 1;
-    if (gi == 0 && col >= 1) g1 = o - 1;
-    if (gj == ny - 1 && row + 1 < NR) g2 = o + HQ;
-    if (gj == 0 && row >= 1) g2 = o - HQ;
-    const bool id = pinned ? (gj == 0 && gi == 0) : (gj == 0 || gj == ny - 1 || gi == 0 || gi == nx - 1);
-    return (unsigned)g1 | ((unsigned)g2 << 15) | (id ? 0x80000000u : 0u) | ((g1 != o || g2 != o) ? 0x40000000u : 0u);
+  // The operator's sign is folded into 1/dx^2, 1/dy^2 (round-to-nearest is
+  // sign-symmetric). Identity rows (the pinned cell; the Dirichlet boundary)
+  // return the cell's value.
+  const bool pinned = __builtin_amdgcn_readfirstlane(C.op) == 0, jac = __builtin_amdgcn_readfirstlane(C.jacobi) != 0;
+  const float scx = uniform(pinned ? -A.cx : A.cx), scy = uniform(pinned ? -A.cy : A.cy);
+  auto lap = [&](const float* L, float c, int oe, int ow, int on, int os) -> float {
+    return __fmul_rn((L[oe] - c) - (c - L[ow]), scx) + __fmul_rn((L[on] - c) - (c - L[os]), scy);
   };
-  static_assert(NR * HQ < (1 << 15), "LDS offsets fit 15 bits");
-  auto put = [&](float* L, int o, unsigned code, float v) {
-    L[o] = v;
-    if (code & 0x40000000u) {
-      L[code & 0x7fffu] = v;
-      L[(code >> 15) & 0x7fffu] = v;
-    }
-  };
-  auto opv = [&](const float* L, int o, unsigned code) -> float {
-    const float c = L[o];
-    const float t = __fmul_rn((L[o + 1] - c) - (c - L[o - 1]), scx) + __fmul_rn((L[o + HQ] - c) - (c - L[o - HQ]), scy);
-    return (code & 0x80000000u) ? c : t;
-  };
-  // Pass 1: every global load of the thread, unconditional (out-of-range
-  // lanes read cell 0 and discard it).
-  float ro[M], po[M];
+  // Pass 1: every global load of the thread, unconditional (cells outside the
+  // domain read its last row or column; their values reach no other cell).
+  const int o0 = (wave + 4) * HQ + li + 4;  // LDS word of the first cell; cell m at o0 + m * TP
+  const int oE = o0 + ((i + 1 < nx) ? 1 : 0), oW = o0 - ((i > 0) ? 1 : 0);
+  const bool inx = i < nx;
+  const unsigned ic = (unsigned)min(i, nx - 1);
+  float ro[M], po[M], mo[M];
   XT xo[M];
-  bool in[M];
+  unsigned idm = 0;           // identity rows (bit m)
+  unsigned inr = 0, egN = 0;  // wave-uniform: row m is in the domain; is its last row
+  const unsigned egS = (wave == 0 && j0 == 0) ? 1u : 0u;
+  const bool bcol = i == 0 || i == nx - 1;
 #pragma unroll
   for (int m = 0; m < M; ++m) {
-    const int j = j0 + TY * m + lj;
-    in[m] = (i < nx) && (j < ny);
-    const size_t k = in[m] ? (size_t)j * nx + i : 0;
-    const float rv = R[k], pv = Pold[k];
-    const XT xv = X[k];
-    ro[m] = in[m] ? rv : 0.f;
-    po[m] = (in[m] && !init) ? pv : 0.f;
-    xo[m] = in[m] ? xv : XT(0);
+    const int j = j0 + TY * m + wave;
+    const size_t row = (size_t)min(j, ny - 1) * nx;
+    ro[m] = (R + row)[ic];
+    po[m] = (Pold + row)[ic];
+    xo[m] = (X + row)[ic];
+    if (j < ny) inr |= 1u << m;
+    if (j == ny - 1) egN |= 1u << m;
+    const bool brow = j == 0 || j == ny - 1;
+    mo[m] = (!jac || brow || bcol) ? 1.0f : A.minvf;
+    if (pinned ? (j == 0 && i == 0) : (brow || bcol)) idm |= 1u << m;
   }
-  float fr[NS], fp[NS];
-  int fo[NS];
-  unsigned fc[NS];
-  bool fin[NS];
+  const bool edges = (egS | egN) != 0;
+  const bool any_id = __any(idm != 0);
+  const bool full = (i0 + TX <= nx) && (j0 + RH <= ny);
+  // Frame: f0 its LDS word, the words of its neighbours, flags (bit 0 in the
+  // domain, 1 identity row), Jacobi weight.
+  float fr[2], fp[2], fw[2];
+  int fo[2], fE = 0, fW = 0, fN = 0, fS = 0;
+  bool fin[2], fid = false;
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const int q = tid + s * NTH;
-    int row = 0, col = 0;
-    if (q < F4) ca_frame_cell(RH, q, row, col);
-    fo[s] = row * HQ + col;
+  for (int s = 0; s < 2; ++s) {
+    const unsigned q = s ? F.b : F.a;
+    const int row = (int)(q >> 8), col = (int)(q & 255u);
     const int gj = j0 + row - 4, gi = i0 + col - 4;
-    fin[s] = (q < F4) && gi >= 0 && gi < nx && gj >= 0 && gj < ny;
-    fc[s] = fin[s] ? code_of(gj, gi, row, col) : 0;
-    const size_t kk = fin[s] ? (size_t)gj * nx + gi : 0;
-    const float rv = R[kk], pv = Pold[kk];
-    fr[s] = fin[s] ? rv : 0.f;
-    fp[s] = (fin[s] && !init) ? pv : 0.f;
+    fin[s] = q != ~0u && gi >= 0 && gi < nx && gj >= 0 && gj < ny;
+    fo[s] = fin[s] ? row * HQ + col : 0;
+    const size_t k = fin[s] ? (size_t)gj * nx + gi : 0;
+    fr[s] = R[k];
+    fp[s] = Pold[k];
+    const bool bnd = gi == 0 || gi == nx - 1 || gj == 0 || gj == ny - 1;
+    fw[s] = (!jac || bnd) ? 1.0f : A.minvf;
+    if (s == 0) {
+      fE = fo[0] + ((gi + 1 < nx) ? 1 : 0);
+      fW = fo[0] - ((gi > 0) ? 1 : 0);
+      fN = fo[0] + ((gj + 1 < ny) ? HQ : 0);
+      fS = fo[0] - ((gj > 0) ? HQ : 0);
+      fid = pinned ? (gj == 0 && gi == 0) : bnd;
+    }
+    if (ca_frame_cells(RH, 4) <= NTH) break;
   }
-  const int o0 = (lj + 4) * HQ + li + 4;  // LDS offset of the thread's first cell; cell m at o0 + m*TY*HQ
-  float mo[M];     // Jacobi weights of the cells
-  unsigned cc[M];  // ghost / identity codes of the cells
+  auto own_put = [&](float* L, int m, float v) {
+    if ((inr >> m) & 1u) L[o0 + m * TP] = v;
+    if (edges) {
+      if ((egN >> m) & 1u) L[o0 + m * TP + HQ] = v;
+      if ((egS >> m) & 1u) L[o0 + m * TP - HQ] = v;
+    }
+  };
+  auto own_lap = [&](const float* L, int m, float c) -> float {
+    const int d = m * TP;
+    float v = lap(L, c, oE + d, oW + d, o0 + d + HQ, o0 + d - HQ);
+    if (any_id) v = ((idm >> m) & 1u) ? c : v;
+    return v;
+  };
+  auto frame_lap = [&](const float* L, float c) -> float {
+    const float v = lap(L, c, fE, fW, fN, fS);
+    return fid ? c : v;
+  };
+  if (init) {
+#pragma unroll
+    for (int m = 0; m < M; ++m) po[m] = 0.f;
+    fp[0] = fp[1] = 0.f;
+  }
 #pragma unroll
   for (int m = 0; m < M; ++m) {
-    const int j = j0 + TY * m + lj;
-    mo[m] = in[m] ? minv_f32(C, A, j, i) : 0.f;
-    cc[m] = in[m] ? code_of(j, i, TY * m + lj + 4, li + 4) : 0;
-    if (in[m]) {
-      put(lP, o0 + m * TY * HQ, cc[m], po[m]);
-      put(lZ, o0 + m * TY * HQ, cc[m], mo[m] * ro[m]);
-    }
+    own_put(lP, m, po[m]);
+    own_put(lZ, m, mo[m] * ro[m]);
   }
-  float fm0 = 0.f;
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    if (fin[s]) {
-      const int row = fo[s] / HQ, col = fo[s] - row * HQ;
-      const float fm = minv_f32(C, A, j0 + row - 4, i0 + col - 4);
-      if (s == 0) fm0 = fm;
-      put(lP, fo[s], fc[s], fp[s]);
-      put(lZ, fo[s], fc[s], fm * fr[s]);
-    }
+  if (fin[0]) {
+    lP[fo[0]] = fp[0];
+    lZ[fo[0]] = fw[0] * fr[0];
+  }
+  if (ca_frame_cells(RH, 4) > NTH && fin[1]) {
+    lP[fo[1]] = fp[1];
+    lZ[fo[1]] = fw[1] * fr[1];
   }
   __syncthreads();
   // Pass 2: a = A p.
   float ao[M];
 #pragma unroll
   for (int m = 0; m < M; ++m) {
-    ao[m] = 0.f;
-    if (in[m]) {
-      ao[m] = opv(lP, o0 + m * TY * HQ, cc[m]);
-      put(lMA, o0 + m * TY * HQ, cc[m], mo[m] * ao[m]);
-    }
+    ao[m] = own_lap(lP, m, po[m]);
+    own_put(lMA, m, mo[m] * ao[m]);
   }
   float fa = 0.f;
   if (tid < F3 && fin[0]) {
-    fa = opv(lP, fo[0], fc[0]);
-    put(lMA, fo[0], fc[0], fm0 * fa);
+    fa = frame_lap(lP, fp[0]);
+    lMA[fo[0]] = fw[0] * fa;
   }
   __syncthreads();
   // Pass 3: the two steps.
-  float r2o[M];
+  float r2o[M], p2o[M];
 #pragma unroll
   for (int m = 0; m < M; ++m) {
-    r2o[m] = 0.f;
-    if (in[m]) {
-      const int o = o0 + m * TY * HQ;
-      const float cv = opv(lMA, o, cc[m]);
-      const float ev = opv(lZ, o, cc[m]);
-      const CaCell v = ca_steps(A, mo[m], ro[m], po[m], ao[m], cv, ev);
-      const size_t k = (size_t)(j0 + TY * m + lj) * nx + i;
+    const float cv = own_lap(lMA, m, mo[m] * ao[m]);
+    const float ev = own_lap(lZ, m, mo[m] * ro[m]);
+    const CaCell v = ca_steps(A, mo[m], ro[m], po[m], ao[m], cv, ev);
+    if (((inr >> m) & 1u) && (full || inx)) {
+      const size_t row = (size_t)(j0 + TY * m + wave) * nx;
       // Streaming stores: the lines are next read in the next round.
-      pcg_store(v.p2, &Pn[k]);
+      pcg_store(v.p2, Pn + row + ic);
       if (!init) {
-        pcg_store(v.r2, &Rn[k]);
+        pcg_store(v.r2, Rn + row + ic);
         if constexpr (XD)
-          pcg_store((xo[m] + A.ca0 * (double)po[m]) + A.ca1 * (double)v.p1, &X[k]);
+          pcg_store((xo[m] + A.ca0 * (double)po[m]) + A.ca1 * (double)v.p1, X + row + ic);
         else
-          pcg_store((xo[m] + A.ca0f * po[m]) + A.ca1f * v.p1, &X[k]);
+          pcg_store((xo[m] + A.ca0f * po[m]) + A.ca1f * v.p1, X + row + ic);
       }
-      r2o[m] = v.r2;
-      put(lP2, o, cc[m], v.p2);
-      put(lZ2, o, cc[m], v.z2);
     }
+    r2o[m] = v.r2;
+    p2o[m] = v.p2;
+    own_put(lP2, m, v.p2);
+    own_put(lZ2, m, v.z2);
   }
   if (tid < F2 && fin[0]) {
-    const float cv = opv(lMA, fo[0], fc[0]);
-    const float ev = opv(lZ, fo[0], fc[0]);
-    const CaCell v = ca_steps(A, fm0, fr[0], fp[0], fa, cv, ev);
-    put(lP2, fo[0], fc[0], v.p2);
-    put(lZ2, fo[0], fc[0], v.z2);
+    const float cv = frame_lap(lMA, fw[0] * fa);
+    const float ev = frame_lap(lZ, fw[0] * fr[0]);
+    const CaCell v = ca_steps(A, fw[0], fr[0], fp[0], fa, cv, ev);
+    lP2[fo[0]] = v.p2;
+    lZ2[fo[0]] = v.z2;
+    fp[0] = v.p2;
   }
   __syncthreads();
   // Pass 4: a' = A p_k+2 (lMA is rewritten: pass 3's reads of it are done).
-  float a2o[M];
 #pragma unroll
   for (int m = 0; m < M; ++m) {
-    a2o[m] = 0.f;
-    if (in[m]) {
-      a2o[m] = opv(lP2, o0 + m * TY * HQ, cc[m]);
-      put(lMA, o0 + m * TY * HQ, cc[m], mo[m] * a2o[m]);
-    }
+    ao[m] = own_lap(lP2, m, p2o[m]);
+    own_put(lMA, m, mo[m] * ao[m]);
   }
-  if (tid < F1 && fin[0]) put(lMA, fo[0], fc[0], fm0 * opv(lP2, fo[0], fc[0]));
+  if (tid < F1 && fin[0]) lMA[fo[0]] = fw[0] * frame_lap(lP2, fp[0]);
   __syncthreads();
   // Pass 5: partials of the new basis at the cells. Products of two floats
   // are exact in FP64, so each fma equals the product followed by the sum.
 #pragma unroll
   for (int m = 0; m < M; ++m) {
-    if (in[m]) {
-      const int o = o0 + m * TY * HQ;
-      const float cv = opv(lMA, o, cc[m]);
-      const float ev = opv(lZ2, o, cc[m]);
-      const double p2 = lP2[o], z2 = lZ2[o], r2 = r2o[m], a2 = a2o[m];
-      const double ma2 = mo[m] * a2o[m], c2 = cv, mc2 = mo[m] * cv, e2 = ev, me2 = mo[m] * ev;
-      acc[0] = __fma_rn(p2, a2, acc[0]);     // W01
-      acc[1] = __fma_rn(p2, c2, acc[1]);     // W02
-      acc[2] = __fma_rn(p2, e2, acc[2]);     // W04
-      acc[3] = __fma_rn(a2, ma2, acc[3]);    // W11
-      acc[4] = __fma_rn(a2, mc2, acc[4]);    // W12
-      acc[5] = __fma_rn(a2, z2, acc[5]);     // W13
-      acc[6] = __fma_rn(a2, me2, acc[6]);    // W14
-      acc[7] = __fma_rn(c2, mc2, acc[7]);    // W22
-      acc[8] = __fma_rn(c2, z2, acc[8]);     // W23
-      acc[9] = __fma_rn(c2, me2, acc[9]);    // W24
-      acc[10] = __fma_rn(r2, z2, acc[10]);   // W33
-      acc[11] = __fma_rn(z2, e2, acc[11]);   // W34
-      acc[12] = __fma_rn(e2, me2, acc[12]);  // W44
-      acc[13] = __fma_rn(r2, r2, acc[13]);   // |r|^2
+    float z2f = mo[m] * r2o[m], ma2f = mo[m] * ao[m];
+    float cv = own_lap(lMA, m, ma2f);
+    float ev = own_lap(lZ2, m, z2f);
+    if (!full) {  // cells beyond the domain add zeros
+      const bool in = ((inr >> m) & 1u) && inx;
+      p2o[m] = in ? p2o[m] : 0.0f;
+      r2o[m] = in ? r2o[m] : 0.0f;
+      ao[m] = in ? ao[m] : 0.0f;
+      z2f = in ? z2f : 0.0f;
+      ma2f = in ? ma2f : 0.0f;
+      cv = in ? cv : 0.0f;
+      ev = in ? ev : 0.0f;
     }
+    const double p2 = p2o[m], z2 = z2f, r2 = r2o[m], a2 = ao[m];
+    const double ma2 = ma2f, c2 = cv, mc2 = mo[m] * cv, e2 = ev, me2 = mo[m] * ev;
+    acc[0] = __fma_rn(p2, a2, acc[0]);     // W01
+    acc[1] = __fma_rn(p2, c2, acc[1]);     // W02
+    acc[2] = __fma_rn(p2, e2, acc[2]);     // W04
+    acc[3] = __fma_rn(a2, ma2, acc[3]);    // W11
+    acc[4] = __fma_rn(a2, mc2, acc[4]);    // W12
+    acc[5] = __fma_rn(a2, z2, acc[5]);     // W13
+    acc[6] = __fma_rn(a2, me2, acc[6]);    // W14
+    acc[7] = __fma_rn(c2, mc2, acc[7]);    // W22
+    acc[8] = __fma_rn(c2, z2, acc[8]);     // W23
+    acc[9] = __fma_rn(c2, me2, acc[9]);    // W24
+    acc[10] = __fma_rn(r2, z2, acc[10]);   // W33
+    acc[11] = __fma_rn(z2, e2, acc[11]);   // W34
+    acc[12] = __fma_rn(e2, me2, acc[12]);  // W44
+    acc[13] = __fma_rn(r2, r2, acc[13]);   // |r|^2
   }
 }
 
@@ -2685,21 +2737,21 @@ __device__ __attribute__((always_inline)) inline void round_body_ca(const KArgs&
   A.alpha = st.alpha;
   A.it = st.it;
   A.x_is_b = st.x_is_b;
-  A.par = (phase == PH_CG) ? parity ^ st.flip : parity;
+  A.par = __builtin_amdgcn_readfirstlane((phase == PH_CG) ? parity ^ st.flip : parity);
   A.x0 = (phase == PH_DEFL_B) ? st.dcoef : 0.0;  // FIN reads x[0] in round_cold
-  A.cx = C.cxf;
-  A.cy = C.cyf;
+  A.cx = uniform(C.cxf);
+  A.cy = uniform(C.cyf);
   A.betaf = (float)A.beta;
   A.alphaf = (float)A.alpha;
-  A.minvf = C.invdf;
+  A.minvf = uniform(C.invdf);
   A.dset = st.dsetup;
-  A.ca0f = (float)st.ca0;
-  A.cb0f = (float)st.cb0;
-  A.ca1f = (float)st.ca1;
-  A.cb1f = (float)st.cb1;
-  A.ca_init = (st.ca_inc == 0);
-  A.ca0 = st.ca0;
-  A.ca1 = st.ca1;
+  A.ca0f = uniform((float)st.ca0);
+  A.cb0f = uniform((float)st.cb0);
+  A.ca1f = uniform((float)st.ca1);
+  A.cb1f = uniform((float)st.cb1);
+  A.ca_init = __builtin_amdgcn_readfirstlane(st.ca_inc == 0);
+  A.ca0 = uniform(st.ca0);
+  A.ca1 = uniform(st.ca1);
   double acc[NP] = {0.0, 0.0, 0.0, 0.0};
   const int r0 = MULTI ? b * C.rpw : b;
   const int r1 = MULTI ? min(r0 + C.rpw, C.nreg) : b + 1;
@@ -2709,9 +2761,11 @@ __device__ __attribute__((always_inline)) inline void round_body_ca(const KArgs&
     if constexpr (M == 0) {
       march_ca<XD>(C, A, b, acc);
     } else {
+      CaFrame F = ca_frame<M>();
       for (int r = r0; r < r1; ++r) {
         if (r > r0) __syncthreads();  // the previous region's LDS reads are done
-        region_ca<M, XD>(C, A, r, acc, lds);
+        asm volatile("" : "+v"(F.a), "+v"(F.b));  // what derives from them stays in the loop
+        region_ca<M, XD>(C, A, r, F, acc, lds);
       }
     }
     block_partials_ca(acc, sm, C.part + (size_t)parity * C.nblk * NPS + b, C.nblk);
