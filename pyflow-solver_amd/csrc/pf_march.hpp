@@ -22,7 +22,7 @@
 // would be halo; four do not fit the 128 registers of a 16-wave workgroup.
 // Rounds of a 400-iteration solve, solve start included, regions -> strips:
 // 1040^2 25.9 -> 22.6 us, 1535^2 45.3 -> 31.7, 2048^2 (FP32 iterate) 46.0 -> 36.1,
-// 2560^2 (FP64 iterate) 97.9 -> 63.7, 4096^2 184.7 -> 126.2.
+// 2560^2 (FP64 iterate) 97.9 -> 61.2, 4096^2 184.7 -> 123.5.
 #pragma once
 
 namespace pf {
@@ -41,6 +41,10 @@ __device__ __attribute__((always_inline)) inline float lane_down(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xF, 0xF, true));  // wave_shr:1
 }
 
+// r and p are read again in the next round and stored as usual; an FP64 x goes
+// past the caches both ways (4096^2: 123.5 us a round against 126.5 with every
+// store streaming and 142.3 with none; 2560^2: 61.2, 63.6, 58.2).
+//
 // One strip segment. EDGE: it reads or owns cells on or beyond the domain's
 // boundary, where neighbours are missing, weights are 1, rows may be
 // identity rows, and loads go cell by cell to clamped places.
@@ -92,7 +96,7 @@ __device__ __attribute__((always_inline)) inline void march_strip(const PfCav& C
   auto loadx = [&](int row, XT (&v)[2]) {
     const PF_GLOBAL XT* q = X + (size_t)min(max(row, tlo), thi) * nx;
     if constexpr (XD) {
-      const MD2 d = *at(q, ox, MD2{});
+      const MD2 d = __builtin_nontemporal_load(at(q, ox, MD2{}));
       v[0] = d.x;
       v[1] = d.y;
     } else {
@@ -204,9 +208,9 @@ __device__ __attribute__((always_inline)) inline void march_strip(const PfCav& C
         y1 = (x1 + a0 * p2.y) + a1 * s1.y;
       }
       if (EDGE ? own0 && own1 : own0) {
-        pcg_store(np2, at(Pn + rb, o4, MF2{}));
+        *at(Pn + rb, o4, MF2{}) = np2;
         if (!init) {
-          pcg_store(nr2, at(Rn + rb, o4, MF2{}));
+          *at(Rn + rb, o4, MF2{}) = nr2;
           if constexpr (XD) {
             const MD2 y = {y0, y1};
             pcg_store(y, at(X + rb, ox, MD2{}));
@@ -216,9 +220,9 @@ __device__ __attribute__((always_inline)) inline void march_strip(const PfCav& C
           }
         }
       } else if (EDGE && cut) {
-        pcg_store(np2.x, at(Pn + rb + 1, o4, float{}));
+        *at(Pn + rb + 1, o4, float{}) = np2.x;
         if (!init) {
-          pcg_store(nr2.x, at(Rn + rb + 1, o4, float{}));
+          *at(Rn + rb + 1, o4, float{}) = nr2.x;
           pcg_store(y0, at(X + rb + 1, ox, XT{}));
         }
       }
