@@ -1,8 +1,8 @@
 // Device phase machine of the projection step: per-cell phase bodies, the
 // scalar "tails" that consume a phase's reduced partials, and the round kernel.
 //
-// Cross-workgroup protocol (no fences, no spin-waits)
-// -------------------------------------------------
+// Cross-workgroup protocol (no fences; spin-waits only in resident solves, pf_resident.hpp)
+// -----------------------------------------------------------------------------------------
 // Cavity c is cut into nreg regions of tpb 64x16-cell tiles stacked in y and
 // covered by nblk workgroups; workgroup b owns regions [b*rpw, (b+1)*rpw)
 // (one cell per thread per tile). In round r every workgroup of c
@@ -2468,6 +2468,22 @@ __device__ __attribute__((noinline)) void local_cg(const PfCav* __restrict__ Cg,
 #include "pf_resident.hpp"
 namespace pf {
 
+// A region's round out of line, for kernels whose solves run resident: they
+// come here only for a solve's first basis and where their workgroups did not
+// meet, and inlined it took registers from the resident loop (64-cavity batch 465
+// against 440 ms). Other phases go through it, for one call a kernel instead of two.
+template <int M, int V>
+__device__ __attribute__((noinline)) void region_ca_cold(int phase, const PfCav* __restrict__ Cg, const PhaseArgs A, int b,
+                                                         double (*sm)[NPS], float* lds, double* part_out, int pstride) {
+  if (phase != PH_CG) {
+    round_cold<float, V>(phase, Cg, A, b, sm, part_out, pstride);
+    return;
+  }
+  double acc[NP] = {0.0, 0.0, 0.0, 0.0};
+  region_ca<M, false>(*Cg, A, b, ca_frame<M>(), acc, lds);
+  block_partials_ca(acc, sm, part_out, pstride);
+}
+
 // Body of one round for workgroup b of cavity c. M > 0 (float32 only): the
 // cavity's region height in tiles. (Issuing the PCG region loads at entry,
 // before the phase is known, gained no time and gave wrong results in
@@ -2766,7 +2782,9 @@ __device__ __attribute__((always_inline)) inline void round_body_ca(const KArgs&
   const int r1 = MULTI ? min(r0 + C.rpw, C.nreg) : b + 1;
   // The partials' address is formed after the region loop (from the
   // descriptor again), which keeps it out of the loop's registers.
-  if (__builtin_expect(phase == PH_CG, 1)) {
+  if constexpr (RES) {
+    region_ca_cold<M, V>(phase, Cg, A, b, sm, lds, C.part + (size_t)parity * C.nblk * NPS + b, C.nblk);
+  } else if (__builtin_expect(phase == PH_CG, 1)) {
     if constexpr (M == 0) {
       march_ca<XD>(C, A, b, acc);
     } else {
